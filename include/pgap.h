@@ -120,7 +120,10 @@ pgap_status pgap_prp_batch_mixed(pgap_engine *e, const uint32_t *words, const ui
 pgap_status pgap_sync(pgap_engine *e);
 
 /* Timing of the last PRP launch: device time measured with HIP events on
- * the engine's stream, and the kernel variant used. */
+ * the engine's stream, and the vector kernel variant its width selects.
+ * matrix_tests counts the numbers that ran on the matrix cores instead (one
+ * number per wavefront): small batches, the remainder of large ones, and
+ * every number too wide for one lane. */
 typedef struct {
     double kernel_ms;
     uint32_t digits;            /* digits per number of the variant */
@@ -129,7 +132,7 @@ typedef struct {
     uint32_t launches;
     uint64_t tests;
     uint32_t graph;             /* 1 when the launch replayed a captured hipGraph */
-    uint32_t reserved;
+    uint32_t matrix_tests;
 } pgap_launch_info;
 /* Timing and shape of the last batch launch.  A batch call repeated with
  * exactly the same arguments (variant, buffers, count, bases) is captured

@@ -40,6 +40,20 @@ const Variant *find_variant(int kind, int bits, int radix, int lanes) {
     return best;
 }
 
+static std::vector<MatrixVariant> &matrix_registry() {
+    static std::vector<MatrixVariant> v;
+    return v;
+}
+
+void register_matrix(const MatrixVariant &v) { matrix_registry().push_back(v); }
+
+const MatrixVariant *find_matrix(int kind, int bits) {
+    const MatrixVariant *best = nullptr;
+    for (const MatrixVariant &v : matrix_registry())
+        if (v.kind == kind && v.max_bits >= bits && (!best || v.max_bits < best->max_bits)) best = &v;
+    return best;
+}
+
 // ---- small device helpers ----------------------------------------------
 
 // Max bit length over a row-major batch (atomicMax into *out).
@@ -161,6 +175,40 @@ pgap_status pgap_engine::pick(int kind, uint32_t bits, Choice *out) {
     return PGAP_OK;
 }
 
+// The kernels of a batch.  A one-lane wavefront takes as long for one number
+// as for 64, and the device takes a round of one such wavefront per SIMD
+// (65536 rows) in about the same time whether it is full or nearly empty;
+// on the matrix cores the time follows the rows from two per SIMD on.  So
+// whole rounds run on the one-lane variant and the remainder of up to
+// `limit` rows on the matrix one, where limit is the rows it finishes in
+// the time of a round: a squaring costs a one-lane wavefront about 4.4 cycles
+// for each of its 1.5 L^2 + 7 L instructions and the matrix variant
+// kMatrixCycles of its SIMD.  Measured, a round of the one-lane variant against
+// 64, 4096 and 16384 rows on the matrix cores, in ms: 330 bits 0.31, 0.14,
+// 0.24, -; 705 bits 2.06, 0.35, 0.78, 2.8; 1108 bits 6.25, 0.56, 1.55, 5.5;
+// 2128 bits 41.9, 1.66, 4.8, 16.5 (one row on one lane: 0.26, 1.6, 5.3 and
+// 38 ms).  Numbers too wide for one lane take the matrix variant whatever
+// their count: 20000 of 4247 bits in 86 ms against 200 on 4 lanes each.  Below
+// kMatrixMinBits the set-up of a number on a whole wavefront costs more than
+// its squarings save.  A caller that forces a radix, lanes or an occupancy
+// keeps the lane kernels.
+constexpr int kMatrixMinBits = 256;
+constexpr uint32_t kMatrixCycles[6] = {0, 420, 550, 735, 825, 1150};  // by container
+
+pgap_status pgap_engine::plan(int kind, uint32_t bits, const Bases &bases, Plan *out) {
+    *out = Plan{};
+    pgap_status st;
+    if ((st = pick(kind, select_bits(kind, bits, bases), &out->lane))) return st;
+    if (opt.radix || opt.lanes_per_number || opt.waves_per_simd > 0 || (int)bits < kMatrixMinBits) return PGAP_OK;
+    out->mx = find_matrix(kind, (int)bits);
+    if (!out->mx || out->lane.v->lanes != 1) return PGAP_OK;
+    const int blocks = std::min(out->mx->blocks, 5);
+    const uint64_t L = (uint64_t)out->lane.v->digits, simds = 4ull * (uint64_t)num_cus;
+    out->round = (uint32_t)(64 * simds);
+    out->limit = (uint32_t)(simds * (3 * L * L / 2 + 7 * L) * 44 / 10 / kMatrixCycles[blocks]);
+    return PGAP_OK;
+}
+
 // Rows whose verdict is 1: the numbers a later strong-PRP base still tests.
 __global__ void select_kernel(const uint8_t *__restrict__ verdict, uint32_t count, uint32_t *__restrict__ sel,
                               uint32_t *__restrict__ nsel) {
@@ -174,44 +222,71 @@ __global__ void zero_kernel(uint32_t *__restrict__ p) {
     if (threadIdx.x == 0) *p = 0;
 }
 
+// nsel[1] = the first of *nsel selected rows that the matrix variant tests
+// (Plan::lane_rows).
+__global__ void split_kernel(uint32_t *__restrict__ nsel, uint32_t round, uint32_t limit) {
+    if (threadIdx.x) return;
+    const uint32_t n = *nsel, rest = round ? n % round : n;
+    nsel[1] = !round || rest <= limit ? n - rest : n;
+}
+
 // Several strong-PRP bases: the first on every row, each later one only on
 // the rows that passed so far (selected on the device), so lanes that
 // already failed do not ride along through the later bases.  Every launch
 // tests one base (the kernels' contract).
-// `sel` (a row index per number of a chunk) and `nsel` (one counter) are the
+// `sel` (a row index per number of a chunk) and `nsel` (two counters) are the
 // survivor scratch, used when several bases are asked for.
-hipError_t pgap_engine::enqueue_batch(const Choice &c, const uint32_t *d_n, uint32_t limbs, size_t count,
+hipError_t pgap_engine::enqueue_batch(const Plan &c, const uint32_t *d_n, uint32_t limbs, size_t count,
                                       const Bases &bases, uint8_t *d_out, uint32_t *sel, uint32_t *nsel,
                                       uint32_t *launches) {
-    const Variant *v = c.v;
+    const Variant *v = c.lane.v;
     const size_t chunk = kBatchChunk;  // grid dimensions are 32-bit: split very large batches
     const uint32_t nb = v->kind == KIND_SPRP ? bases.n : 1;
     Bases first = bases;
     if (v->kind == KIND_SPRP) first.n = 1;
     hipError_t e;
     for (size_t off = 0; off < count; off += chunk) {
-        const uint32_t n = (uint32_t)std::min(chunk, count - off);
+        const uint32_t n = (uint32_t)std::min(chunk, count - off), lane = (uint32_t)c.lane_rows(n);
         const uint32_t *dn = d_n + off * limbs;
         uint8_t *dout = d_out + off;
-        if ((e = v->launch(dn, limbs, n, nullptr, nullptr, first, dout, c.cap, stream)) != hipSuccess) return e;
-        ++*launches;
+        if (lane) {
+            if ((e = v->launch(dn, limbs, lane, nullptr, nullptr, first, dout, c.lane.cap, stream)) != hipSuccess)
+                return e;
+            ++*launches;
+        }
+        if (lane < n) {
+            if ((e = c.mx->launch(dn, limbs, lane, n, nullptr, nullptr, nullptr, first.b[0], dout, stream)) !=
+                hipSuccess)
+                return e;
+            ++*launches;
+        }
         for (uint32_t k = 1; k < nb; ++k) {
             Bases one{};
             one.n = 1;
             one.b[0] = bases.b[k];
             hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, stream, nsel);
             hipLaunchKernelGGL(select_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, dout, n, sel, nsel);
+            if (c.mx) hipLaunchKernelGGL(split_kernel, dim3(1), dim3(64), 0, stream, nsel, c.round, c.limit);
             if ((e = hipGetLastError()) != hipSuccess) return e;
-            if ((e = v->launch(dn, limbs, n, nsel, sel, one, dout, c.cap, stream)) != hipSuccess) return e;
-            ++*launches;
+            if (!c.mx || c.round) {
+                if ((e = v->launch(dn, limbs, n, c.mx ? nsel + 1 : nsel, sel, one, dout, c.lane.cap, stream)) !=
+                    hipSuccess)
+                    return e;
+                ++*launches;
+            }
+            if (c.mx) {
+                if ((e = c.mx->launch(dn, limbs, 0, n, nsel + 1, nsel, sel, one.b[0], dout, stream)) != hipSuccess)
+                    return e;
+                ++*launches;
+            }
         }
     }
     return hipSuccess;
 }
 
-pgap_status pgap_engine::launch_batch(const Choice &c, const uint32_t *d_n, uint32_t limbs, size_t count,
+pgap_status pgap_engine::launch_batch(const Plan &c, const uint32_t *d_n, uint32_t limbs, size_t count,
                                       const Bases &bases, uint8_t *d_out) {
-    const Variant *v = c.v;
+    const Variant *v = c.lane.v;
     if (v->kind == KIND_SPRP && bases.n > 1) {
         pgap_status st;
         if ((st = ensure(d_sel, std::min(count, kBatchChunk) * 4, "survivor index")) ||
@@ -220,12 +295,13 @@ pgap_status pgap_engine::launch_batch(const Choice &c, const uint32_t *d_n, uint
     }
     BatchGraph key;
     key.v = v;
+    key.mx = c.mx;
     key.d_n = d_n;
     key.limbs = limbs;
     key.count = count;
     key.bases = bases;
     key.d_out = d_out;
-    key.cap = c.cap;
+    key.cap = c.lane.cap;
     key.sel = d_sel.p;
     key.nsel = d_nsel.p;
     const bool repeat = graph.same(key);
@@ -276,6 +352,7 @@ pgap_status pgap_engine::launch_batch(const Choice &c, const uint32_t *d_n, uint
     last.lanes_per_number = (uint32_t)v->lanes;
     last.launches = launches;
     last.tests = count;
+    last.matrix_tests = (uint32_t)std::min<size_t>(count - c.lane_rows(count), 0xffffffffu);
     last.graph = replayed ? 1u : 0u;
     last.kernel_ms = -1.0;
     timing_pending = true;
@@ -297,7 +374,7 @@ __global__ void two_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint3
 // Baillie-PSW: the strong base-2 test on every row, the strong Lucas test on
 // the rows that passed (selected on the device into `sel` / `nsel`), then 2
 // itself.
-hipError_t pgap_engine::enqueue_bpsw(const Choice &cs, const Choice &cl, const uint32_t *d_n, uint32_t limbs,
+hipError_t pgap_engine::enqueue_bpsw(const Plan &cs, const Choice &cl, const uint32_t *d_n, uint32_t limbs,
                                      size_t count, uint8_t *d_out, uint32_t *sel, uint32_t *nsel,
                                      uint32_t *launches) {
     Bases two{}, none{};
@@ -308,19 +385,19 @@ hipError_t pgap_engine::enqueue_bpsw(const Choice &cs, const Choice &cl, const u
         const uint32_t n = (uint32_t)std::min(kBatchChunk, count - off);
         const uint32_t *dn = d_n + off * limbs;
         uint8_t *dout = d_out + off;
-        if ((e = cs.v->launch(dn, limbs, n, nullptr, nullptr, two, dout, cs.cap, stream)) != hipSuccess) return e;
+        if ((e = enqueue_batch(cs, dn, limbs, n, two, dout, sel, nsel, launches)) != hipSuccess) return e;
         hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, stream, nsel);
         hipLaunchKernelGGL(select_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, dout, n, sel, nsel);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         if ((e = cl.v->launch(dn, limbs, n, nsel, sel, none, dout, cl.cap, stream)) != hipSuccess) return e;
         hipLaunchKernelGGL(two_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, dn, limbs, n, dout);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        *launches += 2;
+        ++*launches;
     }
     return hipSuccess;
 }
 
-pgap_status pgap_engine::launch_bpsw(const Choice &cs, const Choice &cl, const uint32_t *d_n, uint32_t limbs,
+pgap_status pgap_engine::launch_bpsw(const Plan &cs, const Choice &cl, const uint32_t *d_n, uint32_t limbs,
                                      size_t count, uint8_t *d_out) {
     pgap_status st;
     if ((st = ensure(d_sel, std::min(count, kBatchChunk) * 4, "survivor index")) ||
@@ -339,6 +416,7 @@ pgap_status pgap_engine::launch_bpsw(const Choice &cs, const Choice &cl, const u
     last.lanes_per_number = (uint32_t)cl.v->lanes;
     last.launches = launches;
     last.tests = count;
+    last.matrix_tests = (uint32_t)std::min<size_t>(count - cs.lane_rows(count), 0xffffffffu);
     last.graph = 0;
     last.kernel_ms = -1.0;
     timing_pending = true;
@@ -352,13 +430,14 @@ pgap_status pgap_engine::run_batch(pgap_test kind, const Bases &bs, uint32_t bit
     bits = std::max(bits, 2u);
     pgap_status st;
     if (kind == PGAP_BPSW) {
-        Choice cs, cl;
-        if ((st = pick(KIND_SPRP, bits, &cs)) || (st = pick(KIND_LUCAS, bits, &cl))) return st;
+        Plan cs;
+        Choice cl;
+        if ((st = plan(KIND_SPRP, bits, bs, &cs)) || (st = pick(KIND_LUCAS, bits, &cl))) return st;
         return launch_bpsw(cs, cl, d_n, limbs, count, d_out);
     }
     const int k = kind == PGAP_LUCAS ? KIND_LUCAS : (int)kind;
-    Choice v;
-    if ((st = pick(k, select_bits(k, bits, bs), &v))) return st;
+    Plan v;
+    if ((st = plan(k, bits, bs, &v))) return st;
     return launch_batch(v, d_n, limbs, count, bs, d_out);
 }
 
@@ -588,13 +667,14 @@ pgap_status pgap_prp_batch_device_noalloc(pgap_engine *e, uint32_t limbs, const 
     uint32_t launches = 0;
     hipError_t he;
     if (kind == PGAP_BPSW) {
-        Choice cs, cl;
-        if ((st = e->pick(KIND_SPRP, bits, &cs)) || (st = e->pick(KIND_LUCAS, bits, &cl))) return st;
+        Plan cs;
+        Choice cl;
+        if ((st = e->plan(KIND_SPRP, bits, bs, &cs)) || (st = e->pick(KIND_LUCAS, bits, &cl))) return st;
         he = e->enqueue_bpsw(cs, cl, d_n, limbs, count, d_verdict, sel, nsel, &launches);
     } else {
         const int k = kind == PGAP_LUCAS ? KIND_LUCAS : (int)kind;
-        Choice v;
-        if ((st = e->pick(k, select_bits(k, bits, bs), &v))) return st;
+        Plan v;
+        if ((st = e->plan(k, bits, bs, &v))) return st;
         he = e->enqueue_batch(v, d_n, limbs, count, bs, d_verdict, sel, nsel, &launches);
     }
     if (he != hipSuccess) return e->hip_fail(he, "pgap_prp_batch_device_noalloc launch");

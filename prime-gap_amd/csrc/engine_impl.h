@@ -38,10 +38,27 @@ struct Choice {
     int cap = 0;
 };
 
+// How a batch of one test and width runs: whole rounds of the device on the
+// lane variant, the rest on the matrix cores (see plan()).
+struct Plan {
+    Choice lane;
+    const MatrixVariant *mx = nullptr;
+    uint32_t round = 0;  // rows of a round: one wavefront of one-lane numbers per SIMD
+    uint32_t limit = 0;  // remainder of a round up to which the matrix variant is faster
+    // Rows [0, lane_rows(n)) go to the lane variant, the others to the matrix one.
+    size_t lane_rows(size_t n) const {
+        if (!mx) return n;
+        if (!round) return 0;
+        const size_t rest = n % round;
+        return rest <= limit ? n - rest : n;
+    }
+};
+
 // The last batch launch's arguments and, once the same launch has come
 // twice in a row, its captured graph.
 struct BatchGraph {
     const Variant *v = nullptr;
+    const MatrixVariant *mx = nullptr;
     const uint32_t *d_n = nullptr;
     uint32_t limbs = 0;
     size_t count = 0;
@@ -51,7 +68,7 @@ struct BatchGraph {
     void *sel = nullptr, *nsel = nullptr;
     hipGraphExec_t exec = nullptr;
     bool same(const BatchGraph &o) const {
-        if (v != o.v || d_n != o.d_n || limbs != o.limbs || count != o.count || d_out != o.d_out || cap != o.cap ||
+        if (v != o.v || mx != o.mx || d_n != o.d_n || limbs != o.limbs || count != o.count || d_out != o.d_out || cap != o.cap ||
             sel != o.sel || nsel != o.nsel || bases.n != o.bases.n)
             return false;
         for (uint32_t i = 0; i < bases.n; ++i)
@@ -102,10 +119,10 @@ struct pgap_engine {
     pgap::DevBuf d_sel, d_nsel;  // survivors between strong-PRP bases
     pgap::BatchGraph graph;       // steady-state replay of a repeated batch launch
     uint32_t graph_launches = 0;  // kernel launches inside the captured graph
-    hipError_t enqueue_batch(const pgap::Choice &c, const uint32_t *d_n, uint32_t limbs, size_t count,
+    hipError_t enqueue_batch(const pgap::Plan &c, const uint32_t *d_n, uint32_t limbs, size_t count,
                              const pgap::Bases &bases, uint8_t *d_out, uint32_t *sel, uint32_t *nsel,
                              uint32_t *launches);
-    hipError_t enqueue_bpsw(const pgap::Choice &cs, const pgap::Choice &cl, const uint32_t *d_n, uint32_t limbs,
+    hipError_t enqueue_bpsw(const pgap::Plan &cs, const pgap::Choice &cl, const uint32_t *d_n, uint32_t limbs,
                             size_t count, uint8_t *d_out, uint32_t *sel, uint32_t *nsel, uint32_t *launches);
     std::vector<pgap::Family> families;  // appended only by pgap_family (client thread)
     pgap::Scanner *scanner = nullptr;  // owned; released by scan_shutdown()
@@ -126,9 +143,10 @@ struct pgap_engine {
     pgap_status hip_fail(hipError_t e, const char *what);
     pgap_status ensure(pgap::DevBuf &b, size_t bytes, const char *what);
     pgap_status pick(int kind, uint32_t bits, pgap::Choice *out);  // select(), error when none covers
-    pgap_status launch_batch(const pgap::Choice &c, const uint32_t *d_n, uint32_t limbs, size_t count,
+    pgap_status plan(int kind, uint32_t bits, const pgap::Bases &bases, pgap::Plan *out);
+    pgap_status launch_batch(const pgap::Plan &c, const uint32_t *d_n, uint32_t limbs, size_t count,
                              const pgap::Bases &bases, uint8_t *d_out);
-    pgap_status launch_bpsw(const pgap::Choice &cs, const pgap::Choice &cl, const uint32_t *d_n, uint32_t limbs,
+    pgap_status launch_bpsw(const pgap::Plan &cs, const pgap::Choice &cl, const uint32_t *d_n, uint32_t limbs,
                             size_t count, uint8_t *d_out);
     pgap_status run_batch(pgap_test kind, const pgap::Bases &bs, uint32_t bits, const uint32_t *d_n,
                           uint32_t limbs, size_t count, uint8_t *d_out);

@@ -73,6 +73,21 @@ struct Variant {
     int (*scan_blocks_per_cu)() = nullptr;  // occupancy of the scan kernel
 };
 
+// Matrix-core batch launch (one number per wavefront): work items [first,
+// count) of the rows, `first` read from the device when d_first is set and
+// `count` cut to *d_count when d_count is; d_idx as in batch_launch_fn.
+typedef hipError_t (*matrix_launch_fn)(const uint32_t *d_n, uint32_t limbs, uint32_t first, uint32_t count,
+                                       const uint32_t *d_first, const uint32_t *d_count, const uint32_t *d_idx,
+                                       uint32_t base, uint8_t *d_out, hipStream_t stream);
+
+struct MatrixVariant {
+    int blocks;    // 16-word blocks of the number's container (mont_mf.h's KB)
+    int kind;      // Kind
+    int max_bits;  // largest N, whatever the base
+    matrix_launch_fn launch;
+    scan_launch_fn scan = nullptr;  // set on strong-PRP variants
+};
+
 // Width to select a variant with.  Strong PRP multiplies by the base as a
 // scalar: x < 2N becomes x < 2bN, and the next lazy squaring returns < 2N
 // while 4b^2 N < R.  Variants register max_bits for bases up to 8 (N < R/2^8);
@@ -87,6 +102,8 @@ inline uint32_t select_bits(int kind, uint32_t bits, const Bases &b) {
 // Registry: filled by every instantiation unit at library load.
 void register_variant(const Variant &v);
 const Variant *find_variant(int kind, int bits, int radix, int lanes);
+void register_matrix(const MatrixVariant &v);
+const MatrixVariant *find_matrix(int kind, int bits);  // smallest covering one, or null
 size_t variant_count();
 const Variant *variant_at(size_t i);
 

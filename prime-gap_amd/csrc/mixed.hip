@@ -200,6 +200,7 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
     e->last.lanes_per_number = 0;  // per bucket
     e->last.launches = (ntiles[0] ? 1u : 0u) + (ntiles[1] ? 1u : 0u);
     e->last.tests = count;
+    e->last.matrix_tests = 0;
     e->timing_pending = true;
     if ((he = hipMemcpyAsync(verdict, e->d_out.p, count, hipMemcpyDeviceToHost, e->stream)) != hipSuccess ||
         (he = hipStreamSynchronize(e->stream)) != hipSuccess)

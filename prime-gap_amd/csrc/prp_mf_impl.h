@@ -1,0 +1,93 @@
+// prp_mf_impl.h -- batch and scan kernels of the matrix-core tests, one
+// number per wavefront (prp_mf.h); included by the prp_mf_*.hip units.
+//
+// One wavefront per workgroup: a small batch spreads over as many compute
+// units as it has numbers.  A test costs the latency of its squarings, about
+// 1200 cycles each at 1108 bits and 1900 at 2128 (a one-lane wavefront takes
+// 12 and 43 thousand for its 64 numbers), until every SIMD has two wavefronts.
+#pragma once
+#include <algorithm>
+#include "kernels.h"
+#include "prp_mf.h"
+
+namespace pgap {
+
+// Workgroups of a launch whose count only the device knows: two rounds of
+// the wavefronts the widest width keeps resident (2 per SIMD).
+constexpr uint32_t kMatrixBlocks = 4096;
+
+template <int KB, int KIND>
+__device__ __forceinline__ uint32_t prp_mf_test(const uint32_t *__restrict__ nw, uint32_t limbs, uint32_t base,
+                                                uint32_t *lds) {
+    if constexpr (KIND == KIND_FERMAT2)
+        return mf::fermat2<KB>(nw, limbs, lds, threadIdx.x);
+    else
+        return mf::sprp<KB>(nw, limbs, base, lds, threadIdx.x);
+}
+
+template <int KB, int KIND>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+prp_mf_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint32_t first, uint32_t count,
+              const uint32_t *__restrict__ d_first, const uint32_t *__restrict__ d_count,
+              const uint32_t *__restrict__ d_idx, uint32_t base, uint8_t *__restrict__ out) {
+    __shared__ __align__(16) uint32_t lds[mf::buf_words(KB)];
+    const uint32_t cnt = d_count ? min(*d_count, count) : count;
+#pragma unroll 1
+    for (uint32_t i = (d_first ? *d_first : first) + blockIdx.x; i < cnt; i += gridDim.x) {
+        const uint32_t row = d_idx ? d_idx[i] : i;
+        const uint32_t v = prp_mf_test<KB, KIND>(n + (size_t)row * limbs, limbs, base, lds);
+        if (threadIdx.x == 0) out[row] = (uint8_t)v;
+    }
+}
+
+template <int KB, int KIND>
+hipError_t launch_mf(const uint32_t *d_n, uint32_t limbs, uint32_t first, uint32_t count, const uint32_t *d_first,
+                     const uint32_t *d_count, const uint32_t *d_idx, uint32_t base, uint8_t *d_out,
+                     hipStream_t stream) {
+    if (first >= count) return hipSuccess;
+    const uint32_t blocks = d_count ? std::min(count, kMatrixBlocks) : count - first;
+    hipLaunchKernelGGL((prp_mf_kernel<KB, KIND>), dim3(blocks), dim3(64), 0, stream, d_n, limbs, first, count, d_first,
+                       d_count, d_idx, base, d_out);
+    return hipGetLastError();
+}
+
+// Streaming-scan round: confirmation items, then Fermat items.
+template <int KB>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+scan_mf_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint32_t conf_rows, uint32_t conf_max,
+               uint32_t max_items, const uint32_t *__restrict__ ctr, const uint8_t *__restrict__ base,
+               uint8_t *__restrict__ out) {
+    __shared__ __align__(16) uint32_t lds[mf::buf_words(KB)];
+    const uint32_t nc = min(ctr[3], conf_max), nf = min(ctr[0], max_items);
+#pragma unroll 1
+    for (uint32_t i = blockIdx.x; i < nc + nf; i += gridDim.x) {
+        const uint32_t row = i < nc ? i : conf_rows + (i - nc);
+        const uint32_t *nw = n + (size_t)row * limbs;
+        const uint32_t v = i < nc ? mf::sprp<KB>(nw, limbs, base[i], lds, threadIdx.x)
+                                  : mf::fermat2<KB>(nw, limbs, lds, threadIdx.x);
+        if (threadIdx.x == 0) out[row] = (uint8_t)v;
+    }
+}
+
+template <int KB>
+hipError_t launch_scan_mf(const uint32_t *d_n, uint32_t limbs, uint32_t conf_rows, uint32_t conf_max,
+                          uint32_t max_items, const uint32_t *d_ctr, const uint8_t *d_base, uint8_t *d_out, int,
+                          hipStream_t stream) {
+    const uint32_t blocks = std::min(conf_max + max_items, kMatrixBlocks);
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL((scan_mf_kernel<KB>), dim3(blocks), dim3(64), 0, stream, d_n, limbs, conf_rows, conf_max,
+                       max_items, d_ctr, d_base, d_out);
+    return hipGetLastError();
+}
+
+template <int... KBs>
+struct RegisterMF {
+    RegisterMF() {
+        (register_matrix(MatrixVariant{KBs, KIND_FERMAT2, mf::max_bits(KBs), &launch_mf<KBs, KIND_FERMAT2>}), ...);
+        (register_matrix(MatrixVariant{KBs, KIND_SPRP, mf::max_bits(KBs), &launch_mf<KBs, KIND_SPRP>,
+                                       &launch_scan_mf<KBs>}),
+         ...);
+    }
+};
+
+}  // namespace pgap

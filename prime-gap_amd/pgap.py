@@ -92,7 +92,7 @@ class LaunchInfo(ctypes.Structure):
         ("launches", ctypes.c_uint32),
         ("tests", ctypes.c_uint64),
         ("graph", ctypes.c_uint32),
-        ("reserved", ctypes.c_uint32),
+        ("matrix_tests", ctypes.c_uint32),
     ]
 
 

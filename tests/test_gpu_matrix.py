@@ -1,0 +1,61 @@
+"""Matrix-core variants (one number per wavefront, csrc/mont_mf.h) against the
+oracle: widths at the edges of every container, and batches cut between whole
+rounds of the one-lane variant and a remainder on the matrix cores."""
+import random
+
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+import pgap
+
+pytestmark = pytest.mark.gpu
+
+MERSENNE = [521, 607, 1279, 2203, 2281, 3217, 4253, 4423]
+
+
+def check(engine, vals, kind, bases=(), limbs=None):
+    arr = pgap.to_limbs(vals, limbs or max(pgap.limbs_needed(v) for v in vals))
+    got = engine.prp(arr, kind, bases)
+    want = ol.verdicts(arr, kind, bases)
+    bad = np.nonzero(got != want)[0]
+    assert len(bad) == 0, [(hex(vals[i]), int(got[i]), int(want[i])) for i in bad[:5]]
+    return got
+
+
+# containers of 15, 31, ... 143 words take 32 words - 16 bits
+@pytest.mark.parametrize("blocks", range(1, 10))
+def test_container_edges(engine, blocks):
+    top = min(32 * (16 * blocks - 1) - 16, 4466)  # the widest that every base takes
+    rng = random.Random(blocks)
+    vals = [(1 << top) - 1, (1 << top) - 3, (1 << (top - 1)) + 1, (1 << top) - (1 << (top // 2)) - 1]
+    vals += [rng.getrandbits(b) | (1 << (b - 1)) | 1 for b in (top, top, top - 1, top - 15, top - 16, top - 31, 257)]
+    # every word of the quotient at the ends of the balanced range
+    vals += [int.from_bytes(bytes([c]) * (top // 8 - 1), "little") | 1 for c in (0x7F, 0x80, 0x81, 0xFF)]
+    vals += [0, 1, 2, 3, 5, 9, 341, 561, 2047, 3277, 25326001, 3215031751, (1 << 61) - 1, (1 << 89) - 1]
+    vals += [(1 << p) - 1 for p in MERSENNE if p <= top]
+    vals += [3 * ((1 << p) - 1) for p in MERSENNE if p + 2 <= top]
+    limbs = (top + 31) // 32
+    for kind, bases in ((pgap.FERMAT2, ()), (pgap.SPRP, (2,)), (pgap.SPRP, (3, 5)), (pgap.SPRP, (2, 61))):
+        got = check(engine, vals, kind, bases, limbs)
+        assert engine.last_launch().matrix_tests == len(vals)
+        primes = [i for i, v in enumerate(vals) if v in {(1 << p) - 1 for p in MERSENNE}]
+        assert got[primes].all()
+
+
+@pytest.mark.parametrize("kind,bases", [(pgap.FERMAT2, ()), (pgap.SPRP, (3, 7))])
+def test_remainder_of_a_round(engine, kind, bases):
+    # 65536 rows are a round of one-lane wavefronts: one row, and the rows of
+    # a nearly full second round, beyond it
+    rng = random.Random(len(bases))
+    bits = 300
+    vals = [rng.getrandbits(bits) | (1 << (bits - 1)) | 1 for _ in range(4096)]
+    vals[4095] = vals[0] = vals[17] = (1 << 127) - 1
+    vals[1], vals[2], vals[3] = 2047, 4, 1
+    arr = pgap.to_limbs(vals, (bits + 31) // 32)
+    want = ol.verdicts(arr, kind, bases)
+    for count in (65536, 65537, 65536 + 1000, 2 * 65536 - 1):
+        rows = np.resize(arr, (count, arr.shape[1]))
+        got = engine.prp(rows, kind, bases)
+        assert np.array_equal(got, np.resize(want, count)), count
+        assert engine.last_launch().matrix_tests == (count - 65536 if count - 65536 <= 1000 else 0)
