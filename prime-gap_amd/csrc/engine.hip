@@ -199,7 +199,7 @@ pgap_status pgap_engine::plan(int kind, uint32_t bits, const Bases &bases, Plan 
     *out = Plan{};
     pgap_status st;
     if ((st = pick(kind, select_bits(kind, bits, bases), &out->lane))) return st;
-    if (opt.radix || opt.lanes_per_number || opt.waves_per_simd > 0 || (int)bits < kMatrixMinBits) return PGAP_OK;
+    if (forced() || (kind != KIND_LUCAS && (int)bits < kMatrixMinBits)) return PGAP_OK;
     out->mx = find_matrix(kind, (int)bits);
     if (!out->mx || out->lane.v->lanes != 1) return PGAP_OK;
     const int blocks = std::min(out->mx->blocks, 5);
@@ -374,7 +374,7 @@ __global__ void two_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint3
 // Baillie-PSW: the strong base-2 test on every row, the strong Lucas test on
 // the rows that passed (selected on the device into `sel` / `nsel`), then 2
 // itself.
-hipError_t pgap_engine::enqueue_bpsw(const Plan &cs, const Choice &cl, const uint32_t *d_n, uint32_t limbs,
+hipError_t pgap_engine::enqueue_bpsw(const Plan &cs, const Plan &cl, const uint32_t *d_n, uint32_t limbs,
                                      size_t count, uint8_t *d_out, uint32_t *sel, uint32_t *nsel,
                                      uint32_t *launches) {
     Bases two{}, none{};
@@ -389,7 +389,9 @@ hipError_t pgap_engine::enqueue_bpsw(const Plan &cs, const Choice &cl, const uin
         hipLaunchKernelGGL(zero_kernel, dim3(1), dim3(64), 0, stream, nsel);
         hipLaunchKernelGGL(select_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, dout, n, sel, nsel);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        if ((e = cl.v->launch(dn, limbs, n, nsel, sel, none, dout, cl.cap, stream)) != hipSuccess) return e;
+        e = cl.mx ? cl.mx->launch(dn, limbs, 0, n, nullptr, nsel, sel, 0, dout, stream)
+                  : cl.lane.v->launch(dn, limbs, n, nsel, sel, none, dout, cl.lane.cap, stream);
+        if (e != hipSuccess) return e;
         hipLaunchKernelGGL(two_kernel, dim3((n + 255) / 256), dim3(256), 0, stream, dn, limbs, n, dout);
         if ((e = hipGetLastError()) != hipSuccess) return e;
         ++*launches;
@@ -397,7 +399,7 @@ hipError_t pgap_engine::enqueue_bpsw(const Plan &cs, const Choice &cl, const uin
     return hipSuccess;
 }
 
-pgap_status pgap_engine::launch_bpsw(const Plan &cs, const Choice &cl, const uint32_t *d_n, uint32_t limbs,
+pgap_status pgap_engine::launch_bpsw(const Plan &cs, const Plan &cl, const uint32_t *d_n, uint32_t limbs,
                                      size_t count, uint8_t *d_out) {
     pgap_status st;
     if ((st = ensure(d_sel, std::min(count, kBatchChunk) * 4, "survivor index")) ||
@@ -411,9 +413,9 @@ pgap_status pgap_engine::launch_bpsw(const Plan &cs, const Choice &cl, const uin
         return hip_fail(e, "Baillie-PSW launch");
     e = hipEventRecord(ev1, stream);
     if (e != hipSuccess) return hip_fail(e, "hipEventRecord");
-    last.digits = (uint32_t)cl.v->digits;
-    last.radix_bits = (uint32_t)cl.v->radix;
-    last.lanes_per_number = (uint32_t)cl.v->lanes;
+    last.digits = (uint32_t)cl.lane.v->digits;
+    last.radix_bits = (uint32_t)cl.lane.v->radix;
+    last.lanes_per_number = (uint32_t)cl.lane.v->lanes;
     last.launches = launches;
     last.tests = count;
     last.matrix_tests = (uint32_t)std::min<size_t>(count - cs.lane_rows(count), 0xffffffffu);
@@ -430,9 +432,8 @@ pgap_status pgap_engine::run_batch(pgap_test kind, const Bases &bs, uint32_t bit
     bits = std::max(bits, 2u);
     pgap_status st;
     if (kind == PGAP_BPSW) {
-        Plan cs;
-        Choice cl;
-        if ((st = plan(KIND_SPRP, bits, bs, &cs)) || (st = pick(KIND_LUCAS, bits, &cl))) return st;
+        Plan cs, cl;
+        if ((st = plan(KIND_SPRP, bits, bs, &cs)) || (st = plan(KIND_LUCAS, bits, bs, &cl))) return st;
         return launch_bpsw(cs, cl, d_n, limbs, count, d_out);
     }
     const int k = kind == PGAP_LUCAS ? KIND_LUCAS : (int)kind;
@@ -667,9 +668,8 @@ pgap_status pgap_prp_batch_device_noalloc(pgap_engine *e, uint32_t limbs, const 
     uint32_t launches = 0;
     hipError_t he;
     if (kind == PGAP_BPSW) {
-        Plan cs;
-        Choice cl;
-        if ((st = e->plan(KIND_SPRP, bits, bs, &cs)) || (st = e->pick(KIND_LUCAS, bits, &cl))) return st;
+        Plan cs, cl;
+        if ((st = e->plan(KIND_SPRP, bits, bs, &cs)) || (st = e->plan(KIND_LUCAS, bits, bs, &cl))) return st;
         he = e->enqueue_bpsw(cs, cl, d_n, limbs, count, d_verdict, sel, nsel, &launches);
     } else {
         const int k = kind == PGAP_LUCAS ? KIND_LUCAS : (int)kind;

@@ -122,7 +122,7 @@ struct pgap_engine {
     hipError_t enqueue_batch(const pgap::Plan &c, const uint32_t *d_n, uint32_t limbs, size_t count,
                              const pgap::Bases &bases, uint8_t *d_out, uint32_t *sel, uint32_t *nsel,
                              uint32_t *launches);
-    hipError_t enqueue_bpsw(const pgap::Plan &cs, const pgap::Choice &cl, const uint32_t *d_n, uint32_t limbs,
+    hipError_t enqueue_bpsw(const pgap::Plan &cs, const pgap::Plan &cl, const uint32_t *d_n, uint32_t limbs,
                             size_t count, uint8_t *d_out, uint32_t *sel, uint32_t *nsel, uint32_t *launches);
     std::vector<pgap::Family> families;  // appended only by pgap_family (client thread)
     pgap::Scanner *scanner = nullptr;  // owned; released by scan_shutdown()
@@ -143,10 +143,11 @@ struct pgap_engine {
     pgap_status hip_fail(hipError_t e, const char *what);
     pgap_status ensure(pgap::DevBuf &b, size_t bytes, const char *what);
     pgap_status pick(int kind, uint32_t bits, pgap::Choice *out);  // select(), error when none covers
+    bool forced() const { return opt.radix || opt.lanes_per_number || opt.waves_per_simd > 0; }
     pgap_status plan(int kind, uint32_t bits, const pgap::Bases &bases, pgap::Plan *out);
     pgap_status launch_batch(const pgap::Plan &c, const uint32_t *d_n, uint32_t limbs, size_t count,
                              const pgap::Bases &bases, uint8_t *d_out);
-    pgap_status launch_bpsw(const pgap::Plan &cs, const pgap::Choice &cl, const uint32_t *d_n, uint32_t limbs,
+    pgap_status launch_bpsw(const pgap::Plan &cs, const pgap::Plan &cl, const uint32_t *d_n, uint32_t limbs,
                             size_t count, uint8_t *d_out);
     pgap_status run_batch(pgap_test kind, const pgap::Bases &bs, uint32_t bits, const uint32_t *d_n,
                           uint32_t limbs, size_t count, uint8_t *d_out);

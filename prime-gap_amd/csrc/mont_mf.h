@@ -80,6 +80,7 @@ struct Weights {
 // column sum's value over 2^32 (two products of 572 digits: 2^16.2 times mult).
 constexpr uint32_t BIAS = 1u << 18;       // mult 1 or 2
 constexpr uint32_t BIAS_WIDE = 1u << 24;  // mult up to 63
+constexpr uint32_t BIAS_DIV = 1u << 24;   // words plus a multiple below 2^23 of words
 
 template <int KB>
 struct Wave {
@@ -92,6 +93,11 @@ struct Wave {
     v4i ni[KB + 3];  // N^-1 mod R, u = -3 .. KB - 1
 
     __device__ __forceinline__ void init(uint32_t *lds, uint32_t l) {
+        attach(lds, l);
+        for (int i = (int)l; i < buf_words(KB); i += 64) lds[i] = 0;
+        lds_order();
+    }
+    __device__ __forceinline__ void attach(uint32_t *lds, uint32_t l) {
         lane = l;
         buf = lds + PAD;
         const uint32_t m = l & 15u, h = l >> 4;
@@ -103,8 +109,6 @@ struct Wave {
         st_lo = (int)l + last < LW ? buf + l + last : dummy;
         st_hi = (int)l + last >= 1 && (int)l + last <= LW ? buf + l + last - 1 : dummy;
         st_hi0 = l >= 1 ? buf + l - 1 : dummy;
-        for (int i = (int)l; i < buf_words(KB); i += 64) lds[i] = 0;
-        lds_order();
     }
 
     // A fragment u of the number in the buffer.
@@ -274,10 +278,10 @@ struct Wave {
         store_high(p);
     }
 
-    // 1 if the number in the buffer, times R^-1, is 1 mod N, 2 if it is -1,
-    // else 0 (leaves the buffer overwritten).  Its reduction (x + q N) / R is
-    // within 0.51 N of zero, so 1 and -1 show as themselves; x itself adds
-    // less than 2^22 below the rounding word.
+    // 1 if the number in the buffer, times R^-1, is 1 mod N, 2 if it is -1, 3
+    // if it is 0, else 0 (leaves the buffer overwritten).  Its reduction (x +
+    // q N) / R is within 0.51 N of zero, so 1, -1 and 0 show as themselves; x
+    // itself adds less than 2^22 below the rounding word.
     __device__ __forceinline__ uint32_t classify() const {
         v4i hi[T];
         int64_t s[T];
@@ -298,7 +302,7 @@ struct Wave {
         }
         if (__ballot(rest) != 0) return 0;
         const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)p[0], 1);
-        return w0 == 1u ? 1u : (w0 == 0xffu ? 2u : 0u);
+        return w0 == 1u ? 1u : (w0 == 0xffu ? 2u : (w0 == 0u ? 3u : 0u));
     }
 
     // Loads N (odd, b bits, words in n[] in lane order), its inverse mod R,

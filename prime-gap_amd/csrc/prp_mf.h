@@ -73,7 +73,8 @@ __device__ __forceinline__ uint32_t sprp(const uint32_t *__restrict__ nw, uint32
         w.square(mult, bias, p);
         high = true;
     }
-    if (w.classify() != 0) return 1;
+    const uint32_t k0 = w.classify();
+    if (k0 == 1 || k0 == 2) return 1;
 #pragma unroll 1
     for (int c = 1; c < tz; ++c) {
         if (high)

@@ -8,7 +8,7 @@
 #pragma once
 #include <algorithm>
 #include "kernels.h"
-#include "prp_mf.h"
+#include "lucas_mf.h"
 
 namespace pgap {
 
@@ -79,6 +79,41 @@ hipError_t launch_scan_mf(const uint32_t *d_n, uint32_t limbs, uint32_t conf_row
                        max_items, d_ctr, d_base, d_out);
     return hipGetLastError();
 }
+
+// Strong Lucas: two products a step hold twice the fragments, so a wavefront
+// has the SIMD's registers to itself.
+template <int KB>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
+lucas_mf_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint32_t first, uint32_t count,
+                const uint32_t *__restrict__ d_first, const uint32_t *__restrict__ d_count,
+                const uint32_t *__restrict__ d_idx, uint8_t *__restrict__ out) {
+    __shared__ __align__(16) uint32_t lds[2 * mf::buf_words(KB)];
+    const uint32_t cnt = d_count ? min(*d_count, count) : count;
+#pragma unroll 1
+    for (uint32_t i = (d_first ? *d_first : first) + blockIdx.x; i < cnt; i += gridDim.x) {
+        const uint32_t row = d_idx ? d_idx[i] : i;
+        const uint32_t v = mf::strong_lucas<KB>(n + (size_t)row * limbs, limbs, lds, threadIdx.x);
+        if (threadIdx.x == 0) out[row] = (uint8_t)v;
+    }
+}
+
+template <int KB>
+hipError_t launch_lucas_mf(const uint32_t *d_n, uint32_t limbs, uint32_t first, uint32_t count,
+                           const uint32_t *d_first, const uint32_t *d_count, const uint32_t *d_idx, uint32_t,
+                           uint8_t *d_out, hipStream_t stream) {
+    if (first >= count) return hipSuccess;
+    const uint32_t blocks = d_count ? std::min(count, kMatrixBlocks) : count - first;
+    hipLaunchKernelGGL((lucas_mf_kernel<KB>), dim3(blocks), dim3(64), 0, stream, d_n, limbs, first, count, d_first,
+                       d_count, d_idx, d_out);
+    return hipGetLastError();
+}
+
+template <int... KBs>
+struct RegisterLucasMF {
+    RegisterLucasMF() {
+        (register_matrix(MatrixVariant{KBs, KIND_LUCAS, mf::max_bits(KBs), &launch_lucas_mf<KBs>}), ...);
+    }
+};
 
 template <int... KBs>
 struct RegisterMF {

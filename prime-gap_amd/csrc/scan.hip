@@ -58,18 +58,14 @@ constexpr uint32_t FALLBACK_SPAN = 65536;  // offsets screened per append
 constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may allow fewer)
 
 // Latency-first rounds.  A round costs one test's latency whatever it
-// carries, and a group of 8 lanes finishes a wide test sooner than one lane
-// (2128 bits, 2048 numbers: 11.7 against 40.2 ms) at 59% of its throughput.
-// While at most LATENCY_SIDES sides scan, rounds run on the 8-lane variants
-// (when the one-lane variant is wide): many short rounds, each side a
-// shallower window; above the threshold the one-lane rounds take over
-// again.  1511#/2190 with Baillie-PSW confirmation (p50/p99 per m, ms):
-// threshold 1024: 78/138 at 0.3 of capacity, 118/332 at 4900 m/s, 169/265
-// at half of capacity (5.9 k m/s); 2048: 64/124, 123/364, 193/559; 640:
-// 80/139, 164/229, 168/238.
-constexpr uint32_t LATENCY_SIDES = 1024;     // scanning sides at most
-constexpr uint32_t LATENCY_SIDES_ROW = 256;  // ... and at most this many for 16 lanes instead of 8
-constexpr int LATENCY_MIN_DIGITS = 52;       // one-lane variant at least this wide
+// carries.  While at most LATENCY_SIDES sides scan, rounds run one number per
+// wavefront on the matrix cores: many short rounds, each side a shallower
+// window; above the threshold the one-lane rounds take over, which test more
+// numbers a second (at 2128 bits 1.56 against 1.0 M/s, but in rounds of 42 ms)
+// once enough sides share a round that few of its tests run past a prime.
+// Numbers too wide for one lane always run on the matrix cores.
+constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
+constexpr uint32_t MATRIX_WAVES = 4;      // wavefronts per SIMD in a full matrix round
 constexpr uint32_t LUCAS_POOLS = 4;  // Lucas batches that may run at once (a ring)
 
 enum : uint32_t {
@@ -900,33 +896,20 @@ class Scanner {
         return PGAP_OK;
     }
 
-    // The variant for a Lucas batch of tests of up to `bits` bits: one
-    // number per wavefront (a step's three products at once), whatever the
-    // batch size.
-    // Its tests finish soonest, and beside the rounds' grids it also gives
-    // the larger capacity: 1511#/2190 11.3-11.7 k m/s against 9.7-9.8 k
-    // with the 8-lane variant for batches above 256 tests (3001#/2190: 453-467
-    // against 430-439 m/s), at the same latency for the same arrival rate
-    // (p50/p99 125/367 against 122/358 ms at 4900 m/s).
-    pgap_status lucas_choice(uint32_t bits, Choice *c) {
-        const Variant *vw =
-            e->opt.lanes_per_number || e->opt.radix ? nullptr : find_variant(KIND_LUCAS, (int)bits, 28, 64);
-        if (vw) {
-            *c = Choice{vw, 0};
-            return PGAP_OK;
-        }
-        return e->pick(KIND_LUCAS, bits, c);
-    }
-
     // Start pool p (n items, written by the issue step already queued on the
     // round's stream) as a batch on the Lucas stream.
-    pgap_status lucas_launch(uint32_t p, const Choice &c, uint32_t n) {
+    // One number per wavefront on the matrix cores; a forced lane count keeps
+    // that family's variant.
+    pgap_status lucas_launch(uint32_t p, const Plan &c, uint32_t n) {
         Bases none{};
+        const uint32_t *num = d_lnum + (size_t)p * LP * W;
+        uint8_t *verd = d_lverd + (size_t)p * LP;
         hipError_t he;
         if ((he = hipEventRecord(ev_rows, stream)) != hipSuccess ||
             (he = hipStreamWaitEvent(lstream, ev_rows, 0)) != hipSuccess ||
-            (he = c.v->launch(d_lnum + (size_t)p * LP * W, W, n, nullptr, nullptr, none, d_lverd + (size_t)p * LP,
-                              c.cap, lstream)) != hipSuccess ||
+            (he = c.mx ? c.mx->launch(num, W, 0, n, nullptr, nullptr, nullptr, 0, verd, lstream)
+                       : c.lane.v->launch(num, W, n, nullptr, nullptr, none, verd, c.lane.cap, lstream)) !=
+                hipSuccess ||
             (he = hipEventRecord(ev_lucas[p], lstream)) != hipSuccess)
             return e->hip_fail(he, "strong Lucas batch launch");
         lcount[p] = n;
@@ -999,20 +982,9 @@ class Scanner {
         if (conf.n && (st = e->pick(KIND_SPRP, bits, &cc))) return st;
         // sides that will scan this round (m's waiting for confirmations do not)
         const uint32_t sides = (uint32_t)std::min<uint64_t>(2ull * na, (uint64_t)last_scanning + 2ull * admitted_last);
-        if (sides <= LATENCY_SIDES && !e->opt.lanes_per_number && !e->opt.radix) {
-            // wide one-lane numbers move to 8 lanes (16 while very few sides
-            // scan), 4- and 8-lane numbers to 16
-            const bool row = sides <= LATENCY_SIDES_ROW;
-            const int lanes = cf.v->lanes == 1 && cf.v->digits >= LATENCY_MIN_DIGITS ? (row ? 16 : 8)
-                              : cf.v->lanes == 4 || cf.v->lanes == 8                   ? 16
-                                                                                       : 0;
-            const Variant *lf = lanes ? find_variant(KIND_FERMAT2, (int)bits, 28, lanes) : nullptr;
-            const Variant *lc = lanes && conf.n ? find_variant(KIND_SPRP, (int)bits, 28, lanes) : nullptr;
-            if (lf && (!conf.n || (lc && lc->scan))) {
-                cf = Choice{lf, 0};
-                cc = Choice{lc, 0};
-            }
-        }
+        const MatrixVariant *mx = nullptr;  // of the round's strong-PRP and Fermat rows
+        if (!e->forced() && (cf.v->lanes > 1 || sides <= LATENCY_SIDES))
+            mx = find_matrix(conf.n ? KIND_SPRP : KIND_FERMAT2, (int)bits);
         const Variant *vf = cf.v, *vc = cc.v;
         if (vc && !vc->scan) {
             e->set_error("scan: variant radix %d x %d has no scan kernel", vc->radix, vc->digits);
@@ -1032,12 +1004,13 @@ class Scanner {
         // each side still gets a deep window.
         const Variant *vr = vc ? vc : vf;
         int (*occ)() = vc ? vc->scan_blocks_per_cu : vf->blocks_per_cu;
-        const uint32_t per_wave = e->num_cus * 256u / (uint32_t)std::max(1, vr->lanes);
-        const uint32_t resident_full = (uint32_t)std::max(1, occ ? occ() : 1) * per_wave;
+        const uint32_t lanes = mx ? 64u : (uint32_t)std::max(1, vr->lanes);
+        const uint32_t per_wave = e->num_cus * 256u / lanes;
+        const uint32_t resident_full = mx ? MATRIX_WAVES * per_wave : (uint32_t)std::max(1, occ ? occ() : 1) * per_wave;
         const uint32_t resident = 4ull * sides >= per_wave ? resident_full : std::min(resident_full, per_wave);
-        const uint32_t cpad = 64u / (uint32_t)std::max(1, vr->lanes);  // items per wavefront
+        const uint32_t cpad = 64u / lanes;  // items per wavefront
 
-        Choice lc;
+        Plan lc;
         uint32_t lres = 0, lpool_now = 0, nluc = 0;
         uint64_t issued = 0;
         if (lucas && lbusy == LUCAS_POOLS) {
@@ -1071,8 +1044,8 @@ class Scanner {
                 return e->hip_fail(he, "scan count");
             nluc = h_ctr[6];
             if (nluc) {
-                if ((st = lucas_choice(bits, &lc))) return st;
-                lres = resident < resident_full ? (uint32_t)lc.v->lanes : 0u;
+                if ((st = e->plan(KIND_LUCAS, bits, none, &lc))) return st;
+                lres = resident < resident_full ? (lc.mx ? 64u : (uint32_t)lc.lane.v->lanes) : 0u;
             }
         }
         hipLaunchKernelGGL(issue_kernel, dim3((2 * na + 255) / 256), b256, 0, stream, d_active, na, d_state, cr,
@@ -1086,7 +1059,11 @@ class Scanner {
         // this round's confirmations start their strong Lucas tests now,
         // beside the grid
         if (nluc && (st = lucas_launch(lpool_now, lc, nluc))) return st;
-        if (vc)
+        if (mx && conf.n)
+            he = mx->scan(d_nbuf, W, cr, cr, maxi, d_ctr, d_base, d_verdict, 0, stream);
+        else if (mx)
+            he = mx->launch(d_nbuf + (size_t)cr * W, W, 0, maxi, nullptr, d_ctr, nullptr, 0, d_verdict + cr, stream);
+        else if (vc)
             he = vc->scan(d_nbuf, W, cr, cr, maxi, d_ctr, d_base, d_verdict, cap_c, stream);
         else
             he = vf->launch(d_nbuf + (size_t)cr * W, W, maxi, d_ctr, nullptr, none, d_verdict + cr, cap_f,

@@ -59,3 +59,29 @@ def test_remainder_of_a_round(engine, kind, bases):
         got = engine.prp(rows, kind, bases)
         assert np.array_equal(got, np.resize(want, count)), count
         assert engine.last_launch().matrix_tests == (count - 65536 if count - 65536 <= 1000 else 0)
+
+
+@pytest.mark.parametrize("blocks", range(1, 10))
+def test_strong_lucas_edges(engine, blocks):
+    # the Lucas chain's set-up (parameter search, 1 / Q, N = 2^b - 1) and its
+    # width bounds, against the oracle and the lane variant's bound of 4472
+    top = min(32 * (16 * blocks - 1) - 16, 4472)
+    rng = random.Random(100 + blocks)
+    vals = list(range(0, 130)) + [5459, 5777, 10877, 16109, 18971, 1093 ** 2, 3511 ** 2, (1 << 61) - 1]
+    vals += [(1 << top) - 1, (1 << top) - 3, (1 << (top - 1)) + 1, (rng.getrandbits(top // 2) | 1) ** 2]
+    vals += [rng.getrandbits(b) | (1 << (b - 1)) | 1 for b in (top, top, top - 15, top - 31)]
+    vals += [(1 << p) - 1 for p in MERSENNE if p <= top] + [3 * ((1 << p) - 1) for p in MERSENNE if p + 2 <= top]
+    # primes whose parameter D is large: N = 1 mod 4 and mod the odd primes below 30, 44 and 60
+    for below in (30, 44, 60):
+        M = 4
+        for p in range(3, below, 2):
+            if all(p % q for q in range(3, p, 2)):
+                M *= p
+        v = 1 + M * rng.getrandbits(min(top, 700) - M.bit_length())
+        while not ol.probab_prime(v):
+            v += M
+        vals.append(v)
+    limbs = (top + 31) // 32
+    got = check(engine, vals, pgap.LUCAS, (), limbs)
+    assert got[-3:].all() and engine.last_launch().matrix_tests == len(vals)
+    check(engine, vals, pgap.BPSW, (), limbs)
