@@ -93,6 +93,11 @@ struct Family {
     // K mod p over the engine's sieve prime table (pgap_sieve)
     uint64_t *d_skmod = nullptr;
     uint64_t skmod_limit = 0;
+    // primes <= 2 SL + 1 (pgap_sieve): nsmall Barrett constants, then the
+    // primes, then K mod p; the first nsmall_wave are below 4096
+    uint64_t *d_small = nullptr;
+    uint32_t nsmall = 0, nsmall_wave = 0;
+    uint64_t small_limit = 0;
 };
 }  // namespace pgap
 
@@ -132,6 +137,7 @@ struct pgap_engine {
     uint64_t *sieve_mu = nullptr;
     size_t sieve_nprimes = 0;
     uint64_t sieve_limit = 0;
+    uint32_t *sieve_stage = nullptr;  // pinned staging of pgap_sieve's lists
     void sieve_shutdown();
 
     pgap::Family *family(int id) {
