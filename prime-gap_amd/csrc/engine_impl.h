@@ -77,6 +77,12 @@ struct BatchGraph {
     }
 };
 
+// A prime of pgap_filter_candidates (family.hip, fixed_high).
+struct FilterPrime {
+    uint64_t phi, mu, off;  // 2^64 (K mod p) / p, 2^64 / p, margin - 2^31 mu
+    uint32_t p, kmod;
+};
+
 // K = P#/d with what the device needs to build and screen m*K + x.
 struct Family {
     uint32_t P = 0, D = 0, SL = 0;
@@ -86,9 +92,7 @@ struct Family {
     // trial-division tables for pgap_filter_candidates (built per limit)
     uint32_t filter_limit = 0;
     size_t nprimes = 0;
-    uint32_t *d_primes = nullptr;
-    uint32_t *d_kmod = nullptr;  // K mod p
-    uint64_t *d_mu = nullptr;    // floor((2^64-1)/p) for Barrett reduction
+    FilterPrime *d_filter = nullptr;
     uint32_t stage_end[2] = {0, 0};  // prime-index ends of the first two filter stages
     // K mod p over the engine's sieve prime table (pgap_sieve)
     uint64_t *d_skmod = nullptr;

@@ -12,17 +12,6 @@
 
 namespace pgap {
 
-// K mod p for every p in the table (Horner over K's words, high to low).
-__global__ void kmod_kernel(const uint32_t *__restrict__ K, uint32_t nk, const uint32_t *__restrict__ primes,
-                            uint32_t np, uint32_t *__restrict__ out) {
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= np) return;
-    const uint64_t p = primes[i];
-    uint64_t r = 0;
-    for (int j = (int)nk - 1; j >= 0; --j) r = ((r << 32) | K[j]) % p;
-    out[i] = (uint32_t)r;
-}
-
 // a mod p with mu = floor((2^64-1)/p): the quotient estimate is at most 2
 // short, so two conditional subtractions finish it.
 __device__ __forceinline__ uint64_t mod_barrett(uint64_t a, uint64_t p, uint64_t mu) {
@@ -32,34 +21,156 @@ __device__ __forceinline__ uint64_t mod_barrett(uint64_t a, uint64_t p, uint64_t
     return r >= p ? r - p : r;
 }
 
-// One stage of the trial-division screen over primes [k0, k1).  Stage 0
-// reads every candidate; later stages read the survivors the previous stage
-// appended to idx_in (count in *n_in), so waves stay dense instead of
-// idling behind the few lanes that survive the small primes.
-__global__ void filter_stage_kernel(const uint64_t *__restrict__ m, const int64_t *__restrict__ x,
-                                    const uint32_t *__restrict__ idx_in, const uint32_t *__restrict__ n_in,
-                                    uint32_t count, const uint32_t *__restrict__ primes,
-                                    const uint32_t *__restrict__ kmod, const uint64_t *__restrict__ mu, uint32_t k0,
-                                    uint32_t k1, int last, uint8_t *__restrict__ keep, uint32_t *__restrict__ idx_out,
-                                    uint32_t *__restrict__ n_out) {
-    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
-    const uint32_t n = idx_in ? *n_in : count;
-    if (t >= n) return;
-    const uint32_t i = idx_in ? idx_in[t] : t;
-    const uint64_t mi = m[i];
-    const int64_t xi = x[i];
-    const uint64_t ax = xi < 0 ? (uint64_t)(-(xi + 1)) + 1u : (uint64_t)xi;
-    for (uint32_t k = k0; k < k1; ++k) {
-        const uint64_t p = primes[k], u = mu[k];
-        const uint64_t mr = mod_barrett(mod_barrett(mi, p, u) * kmod[k], p, u);  // m*K mod p
-        const uint64_t xr = mod_barrett(ax, p, u);
-        const bool hit = xi < 0 ? (mr == xr) : ((mr + xr == p) || (mr == 0 && xr == 0));
-        if (hit) return;  // keep[i] stays 0
+// The trial-division test of N = m*K + x by p in 64-bit fixed point, for m <
+// 2^32 and |x| < 2^31: with phi = 2^64 (K mod p) / p to within two units and mu
+// = 2^64 / p to within one, m phi + x mu mod 2^64 is 2^64 (N mod p) / p to within
+// 2 m + |x| < 2^34 units.  So p can divide N only if that, plus the margin 2^34,
+// has a high word of at most 8: four multiply-adds and a compare instead of
+// three 64-bit Barrett reductions.  For p < 2^28 that is exact: the next
+// residue lies 2^64 / p >= 2^36 units away.  Larger primes pass by chance (9 in
+// 2^32) and the exact residue decides.  off holds the margin less 2^31 mu, so
+// that x + 2^31 enters as an unsigned word.
+constexpr uint64_t kMargin = 1ull << 34;
+constexpr uint32_t kMarginTop = 8;
+constexpr uint32_t kFixedExact = 1u << 28;
+
+__global__ void filter_table_kernel(const uint32_t *__restrict__ K, uint32_t nk, const uint32_t *__restrict__ primes,
+                                    uint32_t np, FilterPrime *__restrict__ out) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= np) return;
+    const uint64_t p = primes[i];
+    uint64_t r = 0;
+    for (int j = (int)nk - 1; j >= 0; --j) r = ((r << 32) | K[j]) % p;  // Horner, high to low
+    const uint64_t mu = ~0ull / p, c = 0 - mu * p;                     // 2^64 = mu p + c
+    FilterPrime f;
+    f.phi = r * mu + (uint64_t)((double)r * (double)c / (double)p);
+    f.mu = mu;
+    f.off = kMargin - (mu << 31);
+    f.p = (uint32_t)p;
+    f.kmod = (uint32_t)r;
+    out[i] = f;
+}
+
+// High word of the fixed-point residue of (m, x + 2^31).
+__device__ __forceinline__ uint32_t fixed_high(uint64_t phi, uint64_t mu, uint64_t off, uint32_t m, uint32_t xs) {
+    const uint64_t lo = (uint64_t)m * (uint32_t)phi + off;
+    const uint64_t lo2 = (uint64_t)xs * (uint32_t)mu + lo;
+    return (uint32_t)(lo2 >> 32) + m * (uint32_t)(phi >> 32) + xs * (uint32_t)(mu >> 32);
+}
+
+__device__ __forceinline__ bool divides(const FilterPrime &f, uint64_t m, int64_t x) {
+    const uint64_t p = f.p, u = f.mu;
+    const uint64_t ax = x < 0 ? (uint64_t)(-(x + 1)) + 1u : (uint64_t)x;
+    const uint64_t mr = mod_barrett(mod_barrett(m, p, u) * f.kmod, p, u);  // m*K mod p
+    const uint64_t xr = mod_barrett(ax, p, u);
+    return x < 0 ? (mr == xr) : ((mr + xr == p) || (mr == 0 && xr == 0));
+}
+
+__device__ __forceinline__ bool fits_fixed(uint64_t m, int64_t x) {
+    return m < (1ull << 32) && x >= -(1ll << 31) && x < (1ll << 31);
+}
+
+// A candidate of the prime-parallel stages: (m, x + 2^31) and its row.
+struct Listed {
+    uint2 *pair;
+    uint32_t *row, *n;
+};
+
+// Appends the flagged threads' candidates, one global atomic per workgroup of
+// 1024 (a counter takes one about every 10 ns: per wavefront, 2^20 candidates
+// spent 0.16 ms of the stage's 0.20 on it).
+__device__ __forceinline__ void append(bool flag, uint2 pair, uint32_t row, const Listed &out) {
+    __shared__ uint32_t total, base;
+    if (threadIdx.x == 0) total = 0;
+    __syncthreads();
+    const uint64_t mask = __ballot(flag);
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t at = 0;
+    if (lane == 0) at = atomicAdd(&total, (uint32_t)__popcll(mask));
+    at = (uint32_t)__shfl((int)at, 0, 64) + (uint32_t)__popcll(mask & ((1ull << lane) - 1));
+    __syncthreads();
+    if (threadIdx.x == 0) base = total ? atomicAdd(out.n, total) : 0u;
+    __syncthreads();
+    if (flag) {
+        out.pair[base + at] = pair;
+        out.row[base + at] = row;
     }
-    if (last) {
-        keep[i] = 1;
+}
+
+// First stage: a thread per candidate over the primes below 2^10 (table
+// [0, k1), which the scalar cache holds).  Survivors are kept and listed for
+// the prime-parallel stages.  A candidate too large for the fixed-point test
+// meets every prime here, exactly.
+__global__ void __launch_bounds__(1024) filter_first_kernel(const uint64_t *__restrict__ m, const int64_t *__restrict__ x,
+                                                            uint32_t count, const FilterPrime *__restrict__ table,
+                                                            uint32_t k1, uint32_t np, uint8_t *__restrict__ keep,
+                                                            Listed out) {
+    const uint32_t i = blockIdx.x * 1024u + threadIdx.x;
+    const uint64_t mi = i < count ? m[i] : 0u;
+    const int64_t xi = i < count ? x[i] : 0;
+    const bool fixed = fits_fixed(mi, xi);
+    const uint32_t m32 = (uint32_t)mi, xs = (uint32_t)(xi + (1ll << 31));
+    bool alive = i < count;
+    if (fixed) {  // four primes share a branch
+        const auto high = [&](uint32_t k) {
+            const FilterPrime f = table[k];
+            return fixed_high(f.phi, f.mu, f.off, m32, xs);
+        };
+        uint32_t k = 0;
+        for (; alive && k + 4 <= k1; k += 4)
+            alive = min(min(high(k), high(k + 1)), min(high(k + 2), high(k + 3))) > kMarginTop;
+        for (; alive && k < k1; ++k) alive = high(k) > kMarginTop;
     } else {
-        idx_out[atomicAdd(n_out, 1u)] = i;
+        for (uint32_t k = 0; alive && k < np; ++k) alive = !divides(table[k], mi, xi);
+    }
+    if (i < count) keep[i] = alive ? 1 : 0;
+    append(alive && fixed, make_uint2(m32, xs), i, out);
+}
+
+// The listed candidates still kept.
+__global__ void __launch_bounds__(1024) filter_compact_kernel(const uint8_t *__restrict__ keep, Listed in, Listed out) {
+    const uint32_t n = *in.n;
+    for (uint32_t c0 = blockIdx.x * 1024u; c0 < n; c0 += gridDim.x * 1024u) {
+        const uint32_t c = c0 + threadIdx.x;
+        const uint2 pair = c < n ? in.pair[c] : make_uint2(0, 0);
+        const uint32_t row = c < n ? in.row[c] : 0u;
+        append(c < n && keep[row], pair, row, out);
+        __syncthreads();
+    }
+}
+
+// The other stages (primes below 2^15, then the rest): a thread per prime of
+// [k0, k1), over the listed candidates (gridDim.y workgroups take groups of
+// eight in turn; the candidates are scalar loads and the eight share a branch).  Of 2^20 pairs of 809#
+// some 57 thousand get here, for 75 thousand primes: 4.3 10^9 tests in 0.52 ms
+// (8.3 10^12 a second, the multiply-add rate); a thread per candidate with
+// Barrett reductions kept 1.3 wavefronts per SIMD busy for 28.0 ms, and the
+// primes below 2^15 for 1.27 ms (0.53 in fixed point, waiting for the table).
+__global__ void __launch_bounds__(256) filter_primes_kernel(const uint2 *__restrict__ pair, const uint32_t *__restrict__ idx,
+                                                          const uint32_t *__restrict__ n_in,
+                                                          const FilterPrime *__restrict__ table, uint32_t k0,
+                                                          uint32_t k1, uint8_t *__restrict__ keep) {
+    const uint32_t k = k0 + blockIdx.x * 256u + threadIdx.x, n = *n_in;
+    if (k >= k1) return;
+    const FilterPrime f = table[k];
+    const auto clear = [&](uint32_t c, uint32_t high) {
+        if (high <= kMarginTop && (f.p < kFixedExact || divides(f, pair[c].x, (int64_t)pair[c].y - (1ll << 31))))
+            keep[idx[c]] = 0;
+    };
+    for (uint32_t c = 8 * blockIdx.y; c < n; c += 8 * gridDim.y) {
+        if (c + 8 > n) {
+            for (uint32_t j = c; j < n; ++j) clear(j, fixed_high(f.phi, f.mu, f.off, pair[j].x, pair[j].y));
+            break;
+        }
+        uint32_t high[8], least = ~0u;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+            high[j] = fixed_high(f.phi, f.mu, f.off, pair[c + j].x, pair[c + j].y);
+            least = min(least, high[j]);
+        }
+        if (least > kMarginTop) continue;
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) clear(c + j, high[j]);
     }
 }
 
@@ -119,11 +230,8 @@ __global__ void build_kernel(const uint32_t *__restrict__ K, uint32_t nk, const 
 using namespace pgap;
 
 static void free_tables(Family &f) {
-    if (f.d_primes) (void)hipFree(f.d_primes);
-    if (f.d_kmod) (void)hipFree(f.d_kmod);
-    if (f.d_mu) (void)hipFree(f.d_mu);
-    f.d_primes = f.d_kmod = nullptr;
-    f.d_mu = nullptr;
+    if (f.d_filter) (void)hipFree(f.d_filter);
+    f.d_filter = nullptr;
     f.filter_limit = 0;
 }
 
@@ -137,31 +245,34 @@ void pgap_engine::families_shutdown() {
 }
 
 static pgap_status family_tables(pgap_engine *e, Family &f, uint32_t limit) {
-    if (f.filter_limit == limit && f.d_primes) return PGAP_OK;
+    if (f.filter_limit == limit && f.d_filter) return PGAP_OK;
     free_tables(f);
-    std::vector<uint32_t> ps = primes_upto(limit);
-    std::vector<uint64_t> mu(ps.size());
-    for (size_t i = 0; i < ps.size(); ++i) mu[i] = UINT64_MAX / ps[i];
+    const std::vector<uint32_t> ps = primes_upto(limit);
     f.stage_end[0] = (uint32_t)(std::lower_bound(ps.begin(), ps.end(), 1u << 10) - ps.begin());
     f.stage_end[1] = (uint32_t)(std::lower_bound(ps.begin(), ps.end(), 1u << 15) - ps.begin());
-    const size_t bytes = std::max<size_t>(ps.size(), 1) * sizeof(uint32_t);
+    const size_t n = std::max<size_t>(ps.size(), 1);
     hipError_t he;
-    if ((he = hipMalloc(&f.d_primes, bytes)) != hipSuccess || (he = hipMalloc(&f.d_kmod, bytes)) != hipSuccess ||
-        (he = hipMalloc(&f.d_mu, 2 * bytes)) != hipSuccess) {
+    pgap_status st;
+    if ((st = e->ensure(e->d_idx0, n * sizeof(uint32_t), "filter primes"))) return st;
+    if ((he = hipMalloc(&f.d_filter, n * sizeof(FilterPrime))) != hipSuccess) {
         (void)hipGetLastError();
+        f.d_filter = nullptr;
         e->set_error("hipMalloc for %zu filter primes: %s", ps.size(), hipGetErrorString(he));
-        free_tables(f);
         return PGAP_E_OOM;
     }
     if (!ps.empty()) {
-        he = hipMemcpyAsync(f.d_primes, ps.data(), ps.size() * sizeof(uint32_t), hipMemcpyHostToDevice, e->stream);
-        if (he == hipSuccess)
-            he = hipMemcpyAsync(f.d_mu, mu.data(), mu.size() * sizeof(uint64_t), hipMemcpyHostToDevice, e->stream);
-        if (he != hipSuccess) return e->hip_fail(he, "upload primes");
-        hipLaunchKernelGGL(kmod_kernel, dim3((uint32_t)((ps.size() + 255) / 256)), dim3(256), 0, e->stream, f.d_K,
-                           (uint32_t)f.K.size(), f.d_primes, (uint32_t)ps.size(), f.d_kmod);
-        if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "kmod kernel");
-        if ((he = hipStreamSynchronize(e->stream)) != hipSuccess) return e->hip_fail(he, "kmod sync");
+        he = hipMemcpyAsync(e->d_idx0.p, ps.data(), ps.size() * sizeof(uint32_t), hipMemcpyHostToDevice, e->stream);
+        if (he == hipSuccess) {
+            hipLaunchKernelGGL(filter_table_kernel, dim3((uint32_t)((ps.size() + 255) / 256)), dim3(256), 0,
+                               e->stream, f.d_K, (uint32_t)f.K.size(), (const uint32_t *)e->d_idx0.p,
+                               (uint32_t)ps.size(), f.d_filter);
+            he = hipGetLastError();
+        }
+        if (he == hipSuccess) he = hipStreamSynchronize(e->stream);
+        if (he != hipSuccess) {
+            free_tables(f);
+            return e->hip_fail(he, "filter primes");
+        }
     }
     f.nprimes = ps.size();
     f.filter_limit = limit;
@@ -259,33 +370,36 @@ pgap_status pgap_filter_candidates(pgap_engine *e, int family, const uint64_t *m
     pgap_status st;
     if ((st = family_tables(e, *f, limit))) return st;
     if ((st = e->ensure(e->d_m, count * 8, "m")) || (st = e->ensure(e->d_x, count * 8, "x")) ||
-        (st = e->ensure(e->d_keep, count, "keep")) || (st = e->ensure(e->d_idx0, count * 4, "index")) ||
-        (st = e->ensure(e->d_idx1, count * 4, "index")) || (st = e->ensure(e->d_small, 64, "counters")))
+        (st = e->ensure(e->d_keep, count, "keep")) || (st = e->ensure(e->d_idx0, count * 12, "index")) ||
+        (st = e->ensure(e->d_idx1, count * 12, "index")) || (st = e->ensure(e->d_small, 64, "counters")))
         return st;
     hipError_t he;
     if ((he = hipMemcpyAsync(e->d_m.p, m, count * 8, hipMemcpyHostToDevice, e->stream)) != hipSuccess ||
         (he = hipMemcpyAsync(e->d_x.p, x, count * 8, hipMemcpyHostToDevice, e->stream)) != hipSuccess ||
-        (he = hipMemsetAsync(e->d_keep.p, 0, count, e->stream)) != hipSuccess ||
         (he = hipMemsetAsync(e->d_small.p, 0, 16, e->stream)) != hipSuccess)
         return e->hip_fail(he, "filter upload");
-    // three stages: primes < 2^10, < 2^15, the rest; survivors are compacted
-    // between stages (counters in d_small[0], d_small[1]).
-    const uint32_t ends[3] = {std::min(f->stage_end[0], (uint32_t)f->nprimes),
-                              std::min(f->stage_end[1], (uint32_t)f->nprimes), (uint32_t)f->nprimes};
-    uint32_t *ctr = (uint32_t *)e->d_small.p;
-    uint32_t *idx[2] = {(uint32_t *)e->d_idx0.p, (uint32_t *)e->d_idx1.p};
-    uint32_t k0 = 0;
-    for (int s = 0; s < 3; ++s) {
-        const bool last = (s == 2);
-        const uint32_t *in = s == 0 ? nullptr : idx[(s - 1) & 1];
-        const uint32_t *n_in = s == 0 ? nullptr : ctr + (s - 1);
-        hipLaunchKernelGGL(filter_stage_kernel, dim3((uint32_t)((count + 255) / 256)), dim3(256), 0, e->stream,
-                           (const uint64_t *)e->d_m.p, (const int64_t *)e->d_x.p, in, n_in, (uint32_t)count,
-                           f->d_primes, f->d_kmod, f->d_mu, k0, ends[s], last ? 1 : 0, (uint8_t *)e->d_keep.p,
-                           last ? nullptr : idx[s & 1], last ? nullptr : ctr + s);
-        if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "filter kernel");
-        k0 = ends[s];
+    // primes < 2^10, < 2^15, the rest; survivors are compacted between them
+    // (counters in d_small[0], d_small[1])
+    const uint32_t np = (uint32_t)f->nprimes;
+    const uint32_t e0 = std::min(f->stage_end[0], np), e1 = std::min(f->stage_end[1], np);
+    const auto listed = [&](DevBuf &b, int k) {
+        return Listed{(uint2 *)b.p, (uint32_t *)((uint2 *)b.p + count), (uint32_t *)e->d_small.p + k};
+    };
+    const Listed la = listed(e->d_idx0, 0), lb = listed(e->d_idx1, 1);
+    uint8_t *d_keep = (uint8_t *)e->d_keep.p;
+    hipLaunchKernelGGL(filter_first_kernel, dim3((uint32_t)((count + 1023) / 1024)), dim3(1024), 0, e->stream,
+                       (const uint64_t *)e->d_m.p, (const int64_t *)e->d_x.p, (uint32_t)count, f->d_filter, e0, np,
+                       d_keep, la);
+    if (e0 < e1)
+        hipLaunchKernelGGL(filter_primes_kernel, dim3((e1 - e0 + 255) / 256, 512), dim3(256), 0, e->stream, la.pair,
+                           la.row, la.n, f->d_filter, e0, e1, d_keep);
+    if (e1 < np) {
+        hipLaunchKernelGGL(filter_compact_kernel, dim3((uint32_t)std::min<size_t>((count + 1023) / 1024, 512)),
+                           dim3(1024), 0, e->stream, d_keep, la, lb);
+        hipLaunchKernelGGL(filter_primes_kernel, dim3((np - e1 + 255) / 256, 64), dim3(256), 0, e->stream, lb.pair,
+                           lb.row, lb.n, f->d_filter, e1, np, d_keep);
     }
+    if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "filter kernels");
     if ((he = hipMemcpyAsync(keep, e->d_keep.p, count, hipMemcpyDeviceToHost, e->stream)) != hipSuccess ||
         (he = hipStreamSynchronize(e->stream)) != hipSuccess)
         return e->hip_fail(he, "filter sync");
