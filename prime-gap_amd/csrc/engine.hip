@@ -192,20 +192,22 @@ pgap_status pgap_engine::pick(int kind, uint32_t bits, Choice *out) {
 // kMatrixMinBits the set-up of a number on a whole wavefront costs more than
 // its squarings save.  A caller that forces a radix, lanes or an occupancy
 // keeps the lane kernels.
-constexpr int kMatrixMinBits = 256;
 constexpr uint32_t kMatrixCycles[6] = {0, 420, 550, 735, 825, 1150};  // by container
+
+uint32_t pgap_engine::matrix_limit(int digits, int blocks) const {
+    const uint64_t L = (uint64_t)digits, simds = 4ull * (uint64_t)num_cus;
+    return (uint32_t)(simds * (3 * L * L / 2 + 7 * L) * 44 / 10 / kMatrixCycles[std::min(blocks, 5)]);
+}
 
 pgap_status pgap_engine::plan(int kind, uint32_t bits, const Bases &bases, Plan *out) {
     *out = Plan{};
     pgap_status st;
     if ((st = pick(kind, select_bits(kind, bits, bases), &out->lane))) return st;
-    if (forced() || (kind != KIND_LUCAS && (int)bits < kMatrixMinBits)) return PGAP_OK;
+    if (forced() || (kind != KIND_LUCAS && bits < kMatrixMinBits)) return PGAP_OK;
     out->mx = find_matrix(kind, (int)bits);
     if (!out->mx || out->lane.v->lanes != 1) return PGAP_OK;
-    const int blocks = std::min(out->mx->blocks, 5);
-    const uint64_t L = (uint64_t)out->lane.v->digits, simds = 4ull * (uint64_t)num_cus;
-    out->round = (uint32_t)(64 * simds);
-    out->limit = (uint32_t)(simds * (3 * L * L / 2 + 7 * L) * 44 / 10 / kMatrixCycles[blocks]);
+    out->round = 256u * (uint32_t)num_cus;
+    out->limit = matrix_limit(out->lane.v->digits, out->mx->blocks);
     return PGAP_OK;
 }
 

@@ -38,6 +38,9 @@ struct Choice {
     int cap = 0;
 };
 
+// Narrowest batch for the matrix cores (see plan()).
+constexpr uint32_t kMatrixMinBits = 256;
+
 // How a batch of one test and width runs: whole rounds of the device on the
 // lane variant, the rest on the matrix cores (see plan()).
 struct Plan {
@@ -154,6 +157,8 @@ struct pgap_engine {
     pgap_status ensure(pgap::DevBuf &b, size_t bytes, const char *what);
     pgap_status pick(int kind, uint32_t bits, pgap::Choice *out);  // select(), error when none covers
     bool forced() const { return opt.radix || opt.lanes_per_number || opt.waves_per_simd > 0; }
+    // rows the matrix variant tests in the time of a round of one-lane ones
+    uint32_t matrix_limit(int digits, int blocks) const;
     pgap_status plan(int kind, uint32_t bits, const pgap::Bases &bases, pgap::Plan *out);
     pgap_status launch_batch(const pgap::Plan &c, const uint32_t *d_n, uint32_t limbs, size_t count,
                              const pgap::Bases &bases, uint8_t *d_out);

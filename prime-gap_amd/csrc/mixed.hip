@@ -1,6 +1,6 @@
 // mixed.hip -- pgap_prp_batch_mixed: bucket the numbers, queue tiles widest
-// first and run the persistent kernels of mixed_impl.h (lane-group buckets
-// and one-lane buckets side by side on two streams).
+// first and run the kernels of mixed_impl.h (matrix-core numbers and one-lane
+// buckets side by side on two streams).
 #include <algorithm>
 #include <vector>
 
@@ -74,18 +74,17 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
         e->set_error("pgap_prp_batch_mixed runs FERMAT2 or SPRP (kind %d)", (int)kind);
         return PGAP_E_ARG;
     }
-    // bucket per number: the smallest digit count whose bound covers it, the
-    // one-lane buckets first, then the lane-group ones; headroom below
-    // R = 2^(28 digits): the variants' lazy-reduction bounds (one lane: the
-    // window's; a lane group: 4 or 8 bits)
-    constexpr int N1 = MixedOneLane::n, NB = N1 + MixedGroups::n;
+    // bucket per number: the smallest digit count whose bound covers it,
+    // headroom below R = 2^(28 digits) as the one-lane variants need, or the
+    // last for numbers wider than one lane takes
+    constexpr int N1 = MixedOneLane::n;
     const int slack1 = kind == PGAP_FERMAT2 ? 4 : 8 + (int)(select_bits(KIND_SPRP, 0, bs));
-    const int slack_g = kind == PGAP_FERMAT2 ? 4 : 8;
-    auto max_bits = [&](int b) {
-        return b < N1 ? 28 * MixedOneLane::digits[b] - slack1 : 28 * MixedGroups::digits[b - N1] - slack_g;
+    const int widest = kMixedMaxBits - (kind == PGAP_FERMAT2 ? 4 : 8);
+    struct Bucket {
+        std::vector<uint32_t> rows, bits;
+        uint32_t most = 0;  // widest row
     };
-    auto lanes_of = [&](int b) { return b < N1 ? 1 : MixedGroups::lanes[b - N1]; };
-    std::vector<std::vector<uint32_t>> by_bucket(NB);
+    std::vector<Bucket> bucket(N1 + 1);
     size_t total_words = 0;
     for (size_t i = 0; i < count; ++i) {
         const uint32_t *w = words + offset[i];
@@ -95,35 +94,50 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
                 bits = 32u * (uint32_t)j + (32u - (uint32_t)__builtin_clz(w[j]));
                 break;
             }
+        bits = std::max(bits, 2u);
         int b = 0;
-        while (b < NB && max_bits(b) < (int)std::max(bits, 2u)) ++b;
-        if (b == NB) {
-            e->set_error("pgap_prp_batch_mixed: number %zu has %u bits, above the widest bucket (%d)", i, bits,
-                         max_bits(NB - 1));
+        while (b < N1 && 28 * MixedOneLane::digits[b] - slack1 < (int)bits) ++b;
+        if ((int)bits > widest) {
+            e->set_error("pgap_prp_batch_mixed: number %zu has %u bits, above the widest bucket (%d)", i, bits, widest);
             return PGAP_E_TOO_LARGE;
         }
-        by_bucket[(size_t)b].push_back((uint32_t)i);
+        bucket[(size_t)b].rows.push_back((uint32_t)i);
+        bucket[(size_t)b].bits.push_back(bits);
+        bucket[(size_t)b].most = std::max(bucket[(size_t)b].most, bits);
         total_words = std::max<size_t>(total_words, offset[i] + limbs[i]);
     }
-    // tiles of one wavefront (64 / lanes numbers), widest bucket first, in
-    // two queues: [0] the lane-group kernel's, [1] the one-lane kernel's
-    std::vector<uint32_t> order[2];
-    std::vector<uint8_t> tile_bucket[2];
-    for (int b = NB - 1; b >= 0; --b) {
-        const int q = b < N1 ? 1 : 0;
-        const auto &v = by_bucket[(size_t)b];
-        const size_t per = 64 / (size_t)lanes_of(b);
-        for (size_t k = 0; k < v.size(); k += per) {
-            tile_bucket[q].push_back((uint8_t)(b < N1 ? b : b - N1));
+    // One-lane buckets of more rows than the matrix cores test in the time of
+    // a round go to the persistent kernel in tiles of 64, widest first
+    // (order[1]); the other rows to the matrix cores by container, widest
+    // first (order[0]).
+    std::vector<uint32_t> order[2], container[kMixedContainers];
+    std::vector<uint8_t> tile_bucket;
+    for (int b = N1; b >= 0; --b) {
+        const Bucket &k = bucket[(size_t)b];
+        const MatrixVariant *mx = k.rows.empty() ? nullptr : find_matrix(KIND_FERMAT2, (int)k.most);
+        if (b == N1 || (mx && k.most >= kMatrixMinBits &&
+                        k.rows.size() <= e->matrix_limit(MixedOneLane::digits[b], mx->blocks))) {
+            for (size_t i = 0; i < k.rows.size(); ++i)
+                container[find_matrix(KIND_FERMAT2, (int)k.bits[i])->blocks - 1].push_back(k.rows[i]);
+            continue;
+        }
+        for (size_t i = 0; i < k.rows.size(); i += 64) {
+            tile_bucket.push_back((uint8_t)b);
             for (size_t l = 0; l < 64; ++l)
-                order[q].push_back(l < per && k + l < v.size() ? v[k + l] : 0xffffffffu);
+                order[1].push_back(i + l < k.rows.size() ? k.rows[i + l] : 0xffffffffu);
         }
     }
-    const uint32_t ntiles[2] = {(uint32_t)tile_bucket[0].size(), (uint32_t)tile_bucket[1].size()};
+    MixedEnds ends{};
+    for (int k = kMixedContainers - 1; k >= 0; --k) {
+        order[0].insert(order[0].end(), container[k].begin(), container[k].end());
+        ends.end[k] = (uint32_t)order[0].size();
+    }
+    const uint32_t ntiles = (uint32_t)tile_bucket.size(), nmx = ends.end[0];
+    const bool both = ntiles && nmx;
     (void)hipSetDevice(e->opt.device);
     pgap_status st;
     hipError_t he;
-    // The one-lane kernel runs beside the lane-group kernel on a stream of
+    // The one-lane kernel runs beside the matrix-core kernel on a stream of
     // its own, created for this call and destroyed at its end: a process
     // gets a few hardware queues (GPU_MAX_HW_QUEUES, 4 by default), and a
     // stream kept alive would make the streaming scan's two streams share
@@ -139,14 +153,14 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
             if (ev) (void)hipEventDestroy(ev);
         }
     } aux;
-    if (ntiles[0] && ntiles[1]) {
+    if (both) {
         if ((he = hipStreamCreateWithFlags(&aux.s, hipStreamNonBlocking)) != hipSuccess ||
             (he = hipEventCreateWithFlags(&aux.ev, hipEventDisableTiming)) != hipSuccess)
             return e->hip_fail(he, "mixed stream");
     }
     const size_t b_words = total_words * 4, b_off = count * 8, b_limbs = count * 4;
     const size_t b_order = (order[0].size() + order[1].size()) * 4;
-    if ((st = e->ensure(e->d_n, b_words + b_off + b_limbs + b_order + ntiles[0] + ntiles[1] + 64, "mixed inputs")) ||
+    if ((st = e->ensure(e->d_n, b_words + b_off + b_limbs + b_order + ntiles + 64, "mixed inputs")) ||
         (st = e->ensure(e->d_out, count, "verdicts")) || (st = e->ensure(e->d_small, 64, "tile counters")))
         return st;
     char *base = (char *)e->d_n.p;
@@ -155,9 +169,8 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
     uint32_t *d_limbs = (uint32_t *)((char *)d_off + b_off);
     uint32_t *d_order0 = (uint32_t *)((char *)d_limbs + b_limbs);
     uint32_t *d_order1 = d_order0 + order[0].size();
-    uint8_t *d_tb0 = (uint8_t *)(d_order1 + order[1].size());
-    uint8_t *d_tb1 = d_tb0 + ntiles[0];
-    uint32_t *d_next = (uint32_t *)e->d_small.p;  // [0]: lane-group queue, [1]: one-lane queue
+    uint8_t *d_tb = (uint8_t *)(d_order1 + order[1].size());
+    uint32_t *d_next = (uint32_t *)e->d_small.p;
     if ((he = hipMemcpyAsync(d_words, words, b_words, hipMemcpyHostToDevice, e->stream)) != hipSuccess ||
         (he = hipMemcpyAsync(d_off, offset, b_off, hipMemcpyHostToDevice, e->stream)) != hipSuccess ||
         (he = hipMemcpyAsync(d_limbs, limbs, b_limbs, hipMemcpyHostToDevice, e->stream)) != hipSuccess ||
@@ -165,30 +178,26 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
                                                  hipMemcpyHostToDevice, e->stream)) != hipSuccess) ||
         (order[1].size() && (he = hipMemcpyAsync(d_order1, order[1].data(), order[1].size() * 4,
                                                  hipMemcpyHostToDevice, e->stream)) != hipSuccess) ||
-        (ntiles[0] && (he = hipMemcpyAsync(d_tb0, tile_bucket[0].data(), ntiles[0], hipMemcpyHostToDevice,
-                                           e->stream)) != hipSuccess) ||
-        (ntiles[1] && (he = hipMemcpyAsync(d_tb1, tile_bucket[1].data(), ntiles[1], hipMemcpyHostToDevice,
-                                           e->stream)) != hipSuccess) ||
-        (he = hipMemsetAsync(d_next, 0, 8, e->stream)) != hipSuccess)
+        (ntiles && (he = hipMemcpyAsync(d_tb, tile_bucket.data(), ntiles, hipMemcpyHostToDevice, e->stream)) !=
+                       hipSuccess) ||
+        (he = hipMemsetAsync(d_next, 0, 4, e->stream)) != hipSuccess)
         return e->hip_fail(he, "mixed upload");
-    const MixedLaunch lg_launch{d_words, d_off, d_limbs, d_order0, d_tb0, ntiles[0], d_next, bs, (uint8_t *)e->d_out.p};
-    const MixedLaunch one_launch{d_words, d_off, d_limbs, d_order1, d_tb1, ntiles[1], d_next + 1, bs,
-                                 (uint8_t *)e->d_out.p};
-    // the lane-group kernel (the widest tiles) on the engine's stream, the
+    const MixedLaunch mx{d_words, d_off, d_limbs, d_order0, nullptr, 0, nullptr, bs, (uint8_t *)e->d_out.p};
+    const MixedLaunch one{d_words, d_off, d_limbs, d_order1, d_tb, ntiles, d_next, bs, (uint8_t *)e->d_out.p};
+    // the matrix-core kernel (the widest numbers) on the engine's stream, the
     // one-lane kernel beside it on the second stream; the second joins the
     // first before the end event
     if ((he = hipEventRecord(e->ev0, e->stream)) != hipSuccess) return e->hip_fail(he, "event");
-    const bool both = ntiles[0] && ntiles[1];
-    if (ntiles[0]) {
-        he = kind == PGAP_FERMAT2 ? launch_mixed_lg_fermat(lg_launch, e->opt.device, e->stream)
-                                  : launch_mixed_lg_sprp(lg_launch, e->opt.device, e->stream);
-        if (he != hipSuccess) return e->hip_fail(he, "mixed lane-group kernel");
+    if (nmx) {
+        he = kind == PGAP_FERMAT2 ? launch_mixed_mf_fermat(mx, ends, e->stream)
+                                  : launch_mixed_mf_sprp(mx, ends, e->stream);
+        if (he != hipSuccess) return e->hip_fail(he, "mixed matrix-core kernel");
     }
-    if (ntiles[1]) {
+    if (ntiles) {
         hipStream_t s1 = both ? aux.s : e->stream;
         if (both && (he = hipStreamWaitEvent(s1, e->ev0, 0)) != hipSuccess) return e->hip_fail(he, "mixed stream");
-        he = kind == PGAP_FERMAT2 ? launch_mixed_fermat(one_launch, e->opt.device, s1)
-                                  : launch_mixed_sprp(one_launch, e->opt.device, s1);
+        he = kind == PGAP_FERMAT2 ? launch_mixed_fermat(one, e->opt.device, s1)
+                                  : launch_mixed_sprp(one, e->opt.device, s1);
         if (he != hipSuccess) return e->hip_fail(he, "mixed kernel");
         if (both && ((he = hipEventRecord(aux.ev, s1)) != hipSuccess ||
                      (he = hipStreamWaitEvent(e->stream, aux.ev, 0)) != hipSuccess))
@@ -198,9 +207,9 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
     e->last.digits = 0;
     e->last.radix_bits = 28;
     e->last.lanes_per_number = 0;  // per bucket
-    e->last.launches = (ntiles[0] ? 1u : 0u) + (ntiles[1] ? 1u : 0u);
+    e->last.launches = (nmx ? 1u : 0u) + (ntiles ? 1u : 0u);
     e->last.tests = count;
-    e->last.matrix_tests = 0;
+    e->last.matrix_tests = nmx;
     e->timing_pending = true;
     if ((he = hipMemcpyAsync(verdict, e->d_out.p, count, hipMemcpyDeviceToHost, e->stream)) != hipSuccess ||
         (he = hipStreamSynchronize(e->stream)) != hipSuccess)

@@ -85,3 +85,21 @@ def test_strong_lucas_edges(engine, blocks):
     got = check(engine, vals, pgap.LUCAS, (), limbs)
     assert got[-3:].all() and engine.last_launch().matrix_tests == len(vals)
     check(engine, vals, pgap.BPSW, (), limbs)
+
+
+@pytest.mark.parametrize("kind,bases", [(pgap.FERMAT2, ()), (pgap.SPRP, (2, 61))])
+def test_mixed_batch_on_both_kernels(engine, kind, bases):
+    # a one-lane bucket with more rows than the matrix cores take, beside
+    # buckets of a few rows and one number at every container's width
+    rng = random.Random(7)
+    vals = [rng.getrandbits(300) | (1 << 299) | 1 for _ in range(5000)]
+    vals += [rng.getrandbits(b) | (1 << (b - 1)) | 1 for b in (700, 720, 1100, 2100, 2180, 2250, 4400)]
+    vals += [rng.getrandbits(32 * (16 * k - 1) - 16) | 1 for k in range(1, 9)]
+    vals += [(1 << p) - 1 for p in MERSENNE] + [3 * ((1 << p) - 1) for p in MERSENNE] + [0, 1, 2, 3, 5, 2047, 341]
+    rng.shuffle(vals)
+    got = engine.prp_mixed([pgap.to_limbs([v], pgap.limbs_needed(v))[0] for v in vals], kind, bases)
+    if kind == pgap.FERMAT2:
+        assert 0 < engine.last_launch().matrix_tests < 100
+    want = ol.verdicts(pgap.to_limbs(vals, 140), kind, bases)
+    bad = np.nonzero(got != want)[0]
+    assert len(bad) == 0, [(hex(vals[i])[:40], vals[i].bit_length(), int(got[i]), int(want[i])) for i in bad[:5]]
