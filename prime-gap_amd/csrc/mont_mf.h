@@ -122,9 +122,43 @@ struct Wave {
         f.w = (int)__builtin_amdgcn_perm((uint32_t)v.x, lo, sel);
         return f;
     }
+    // Lane 16 h + 4 g + j of fragment u holds piece u + g of the number (16
+    // words; pieces outside 0 .. KB - 1 are zero), so one load in four is
+    // enough: the fragments between are its rows moved by 4 lanes a step, at
+    // 1 or 2 moves a word against 1.2 words loaded and a permute.  The
+    // kernel is bound by LDS reads (a squaring read 159 cycles of them at 1108
+    // bits, 109 now) as much as by the vector ALU: 3.06 -> 3.90 M tests/s at 1108
+    // bits, 1.0 -> 1.07 at 2128, 237 -> 248 k at 4247.  Moving words for the B
+    // fragments too (2 moves each) costs more than the reads they replace.
     __device__ __forceinline__ void load_a_all(v4i (&a)[KB + 3]) const {
 #pragma unroll
-        for (int u = -3; u < KB; ++u) a[u + 3] = load_a(u);
+        for (int b = 0; b < KB; b += 4) a[b + 3] = load_a(b);
+#pragma unroll
+        for (int u = -3; u < KB; ++u) {
+            if (u >= 0 && u % 4 == 0) continue;
+            const v4i z = {0, 0, 0, 0};
+            if (u < 0) {
+                a[u + 3] = u == -1 ? shift<0x114>(z, a[3]) : u == -2 ? shift<0x118>(z, a[3]) : shift<0x11C>(z, a[3]);
+            } else {
+                const int b = u / 4 * 4, r = u % 4;
+                v4i up = z;
+                if (b + 4 < KB) {
+                    const v4i &f = a[b + 7];
+                    up = r == 1 ? shift<0x11C>(z, f) : r == 2 ? shift<0x118>(z, f) : shift<0x114>(z, f);
+                }
+                const v4i &f = a[b + 3];
+                a[u + 3] = r == 1 ? shift<0x104>(up, f) : r == 2 ? shift<0x108>(up, f) : shift<0x10C>(up, f);
+            }
+        }
+    }
+    // Rows of 16 lanes moved by a DPP shift; lanes without a source keep old.
+    template <int CTRL>
+    __device__ __forceinline__ static int shift(int old, int v) {
+        return __builtin_amdgcn_update_dpp(old, v, CTRL, 0xF, 0xF, false);
+    }
+    template <int CTRL>
+    __device__ __forceinline__ static v4i shift(const v4i &old, const v4i &v) {
+        return v4i{shift<CTRL>(old.x, v.x), shift<CTRL>(old.y, v.y), shift<CTRL>(old.z, v.z), shift<CTRL>(old.w, v.w)};
     }
 
     // Every B fragment of the number in the buffer, for its low or high tiles.
@@ -260,13 +294,13 @@ struct Wave {
         load_b_high(bh);
         load_b_low(bl);
         mul_low(lo, a, bl);
+        // the high columns of T are summed while its low words are carried
+        mul_high<3, KB + 3>(hi, a, bh);
         columns(lo, Weights(1), k_low(BIAS), k_rest(BIAS), s);
         carry(s, p);
         store_low(p);
-        // q = -T N^-1 mod R; the high columns of T are summed while its low
-        // words travel through the buffer
+        // q = -T N^-1 mod R
         load_b_low(bl);
-        mul_high<3, KB + 3>(hi, a, bh);
         mul_low(lo, ni, bl);
         columns(lo, Weights(-1), k_low(BIAS), k_rest(BIAS), s);
         carry(s, p);
