@@ -80,12 +80,20 @@ typedef hipError_t (*matrix_launch_fn)(const uint32_t *d_n, uint32_t limbs, uint
                                        const uint32_t *d_first, const uint32_t *d_count, const uint32_t *d_idx,
                                        uint32_t base, uint8_t *d_out, hipStream_t stream);
 
+// Streaming-scan launch on the matrix cores: strong Lucas tests of the nluc
+// numbers at d_lnum (verdicts at d_lverd) beside the rows of scan_launch_fn,
+// one grid for the round's every test.
+typedef hipError_t (*matrix_scan_fn)(const uint32_t *d_n, uint32_t limbs, uint32_t conf_rows, uint32_t conf_max,
+                                     uint32_t max_items, const uint32_t *d_ctr, const uint8_t *d_base,
+                                     uint8_t *d_out, const uint32_t *d_lnum, uint32_t nluc, uint8_t *d_lverd,
+                                     hipStream_t stream);
+
 struct MatrixVariant {
     int blocks;    // 16-word blocks of the number's container (mont_mf.h's KB)
     int kind;      // Kind
     int max_bits;  // largest N, whatever the base
     matrix_launch_fn launch;
-    scan_launch_fn scan = nullptr;  // set on strong-PRP variants
+    matrix_scan_fn scan = nullptr;  // set on strong-PRP variants
 };
 
 // Width to select a variant with.  Strong PRP multiplies by the base as a

@@ -51,32 +51,45 @@ hipError_t launch_mf(const uint32_t *d_n, uint32_t limbs, uint32_t first, uint32
     return hipGetLastError();
 }
 
-// Streaming-scan round: confirmation items, then Fermat items.
+// Streaming-scan round: strong Lucas items (the longest tests), strong-PRP
+// confirmations, then Fermat items, in one grid.  On a stream of their own the
+// Lucas tests overlap the grid only while the streams have hardware queues of
+// their own: with two engines in a process they shared one, and every round of
+// 1.9 to 5 ms (2128 bits) waited 2.75 ms for its Lucas batch.
 template <int KB>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 scan_mf_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint32_t conf_rows, uint32_t conf_max,
                uint32_t max_items, const uint32_t *__restrict__ ctr, const uint8_t *__restrict__ base,
-               uint8_t *__restrict__ out) {
-    __shared__ __align__(16) uint32_t lds[mf::buf_words(KB)];
+               uint8_t *__restrict__ out, const uint32_t *__restrict__ lnum, uint32_t nluc,
+               uint8_t *__restrict__ lverd) {
+    __shared__ __align__(16) uint32_t lds[2 * mf::buf_words(KB)];
     const uint32_t nc = min(ctr[3], conf_max), nf = min(ctr[0], max_items);
 #pragma unroll 1
-    for (uint32_t i = blockIdx.x; i < nc + nf; i += gridDim.x) {
-        const uint32_t row = i < nc ? i : conf_rows + (i - nc);
-        const uint32_t *nw = n + (size_t)row * limbs;
-        const uint32_t v = i < nc ? mf::sprp<KB>(nw, limbs, base[i], lds, threadIdx.x)
-                                  : mf::fermat2<KB>(nw, limbs, lds, threadIdx.x);
-        if (threadIdx.x == 0) out[row] = (uint8_t)v;
+    for (uint32_t i = blockIdx.x; i < nluc + nc + nf; i += gridDim.x) {
+        uint32_t v;
+        uint8_t *o;
+        if (i < nluc) {
+            v = mf::strong_lucas<KB>(lnum + (size_t)i * limbs, limbs, lds, threadIdx.x);
+            o = lverd + i;
+        } else {
+            const uint32_t r = i - nluc, row = r < nc ? r : conf_rows + (r - nc);
+            const uint32_t *nw = n + (size_t)row * limbs;
+            v = r < nc ? mf::sprp<KB>(nw, limbs, base[r], lds, threadIdx.x)
+                       : mf::fermat2<KB>(nw, limbs, lds, threadIdx.x);
+            o = out + row;
+        }
+        if (threadIdx.x == 0) *o = (uint8_t)v;
     }
 }
 
 template <int KB>
 hipError_t launch_scan_mf(const uint32_t *d_n, uint32_t limbs, uint32_t conf_rows, uint32_t conf_max,
-                          uint32_t max_items, const uint32_t *d_ctr, const uint8_t *d_base, uint8_t *d_out, int,
-                          hipStream_t stream) {
-    const uint32_t blocks = std::min(conf_max + max_items, kMatrixBlocks);
+                          uint32_t max_items, const uint32_t *d_ctr, const uint8_t *d_base, uint8_t *d_out,
+                          const uint32_t *d_lnum, uint32_t nluc, uint8_t *d_lverd, hipStream_t stream) {
+    const uint32_t blocks = std::min(nluc + conf_max + max_items, kMatrixBlocks);
     if (blocks == 0) return hipSuccess;
     hipLaunchKernelGGL((scan_mf_kernel<KB>), dim3(blocks), dim3(64), 0, stream, d_n, limbs, conf_rows, conf_max,
-                       max_items, d_ctr, d_base, d_out);
+                       max_items, d_ctr, d_base, d_out, d_lnum, nluc, d_lverd);
     return hipGetLastError();
 }
 

@@ -66,6 +66,7 @@ constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may a
 // Numbers too wide for one lane always run on the matrix cores.
 constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
 constexpr uint32_t MATRIX_WAVES = 4;      // wavefronts per SIMD in a full matrix round
+constexpr uint32_t MATRIX_WAVES_HELD = 2;  // ... while few sides scan
 constexpr uint32_t LUCAS_POOLS = 4;  // Lucas batches that may run at once (a ring)
 
 enum : uint32_t {
@@ -1007,7 +1008,8 @@ class Scanner {
         const uint32_t lanes = mx ? 64u : (uint32_t)std::max(1, vr->lanes);
         const uint32_t per_wave = e->num_cus * 256u / lanes;
         const uint32_t resident_full = mx ? MATRIX_WAVES * per_wave : (uint32_t)std::max(1, occ ? occ() : 1) * per_wave;
-        const uint32_t resident = 4ull * sides >= per_wave ? resident_full : std::min(resident_full, per_wave);
+        const uint32_t held = mx ? MATRIX_WAVES_HELD * per_wave : per_wave;
+        const uint32_t resident = 4ull * sides >= per_wave ? resident_full : std::min(resident_full, held);
         const uint32_t cpad = 64u / lanes;  // items per wavefront
 
         Plan lc;
@@ -1043,7 +1045,9 @@ class Scanner {
                 (he = hipStreamSynchronize(stream)) != hipSuccess)
                 return e->hip_fail(he, "scan count");
             nluc = h_ctr[6];
-            if (nluc) {
+            if (nluc && mx) {
+                lres = 64;
+            } else if (nluc) {
                 if ((st = e->plan(KIND_LUCAS, bits, none, &lc))) return st;
                 lres = resident < resident_full ? (lc.mx ? 64u : (uint32_t)lc.lane.v->lanes) : 0u;
             }
@@ -1057,10 +1061,12 @@ class Scanner {
                            nrows, d_ctr, d_center, CW, d_lists, CAP, d_nbuf, W);
         if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "scan issue");
         // this round's confirmations start their strong Lucas tests now,
-        // beside the grid
-        if (nluc && (st = lucas_launch(lpool_now, lc, nluc))) return st;
+        // beside the grid (in it, on the matrix cores)
+        const uint32_t *lnum = lucas ? d_lnum + (size_t)lpool_now * LP * W : nullptr;
+        uint8_t *lverd = lucas ? d_lverd + (size_t)lpool_now * LP : nullptr;
+        if (nluc && !mx && (st = lucas_launch(lpool_now, lc, nluc))) return st;
         if (mx && conf.n)
-            he = mx->scan(d_nbuf, W, cr, cr, maxi, d_ctr, d_base, d_verdict, 0, stream);
+            he = mx->scan(d_nbuf, W, cr, cr, maxi, d_ctr, d_base, d_verdict, lnum, nluc, lverd, stream);
         else if (mx)
             he = mx->launch(d_nbuf + (size_t)cr * W, W, 0, maxi, nullptr, d_ctr, nullptr, 0, d_verdict + cr, stream);
         else if (vc)
@@ -1071,6 +1077,12 @@ class Scanner {
         if (he != hipSuccess) return e->hip_fail(he, "scan test launch");
         hipLaunchKernelGGL(retire_kernel, dim3((nrows + 255) / 256), b256, 0, stream, d_items, d_idx, cr, nrows,
                            d_verdict, d_ctr, confirm, d_state);
+        if (nluc && mx) {
+            hipLaunchKernelGGL(lucas_retire_kernel, dim3((nluc + 255) / 256), b256, 0, stream,
+                               d_lpool + (size_t)lpool_now * LP, lverd, nluc, d_state);
+            hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(64), 0, stream, d_lctr + lpool_now);
+            issued += nluc;
+        }
         hipLaunchKernelGGL(update_kernel, dim3((na + 255) / 256), b256, 0, stream, d_active, na, d_state, d_lists,
                            CAP, conf.n + (lucas ? 1u : 0u), d_ctr, d_events);
         if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "scan retire");
