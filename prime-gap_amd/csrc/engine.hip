@@ -185,14 +185,13 @@ pgap_status pgap_engine::pick(int kind, uint32_t bits, Choice *out) {
 // for each of its 1.5 L^2 + 7 L instructions and the matrix variant
 // kMatrixCycles of its SIMD.  Measured, a round of the one-lane variant against
 // 64, 4096 and 16384 rows on the matrix cores, in ms: 330 bits 0.31, 0.14,
-// 0.24, -; 705 bits 2.06, 0.35, 0.78, 2.8; 1108 bits 6.25, 0.56, 1.55, 5.5;
-// 2128 bits 41.9, 1.66, 4.8, 16.5 (one row on one lane: 0.26, 1.6, 5.3 and
-// 38 ms).  Numbers too wide for one lane take the matrix variant whatever
-// their count: 20000 of 4247 bits in 86 ms against 200 on 4 lanes each.  Below
+// 0.24, -; 705 bits 2.1, 0.34, 0.65, 2.4; 1108 bits 6.3, 0.56, 1.3, 4.5; 2128
+// bits 42, 1.65, 4.6, 16.4 (one row on one lane: 0.26, 1.6, 5.3 and 38 ms).  Numbers too wide for one lane take the matrix variant whatever
+// their count: 20000 of 4247 bits in 78 ms against 199 on 4 lanes each.  Below
 // kMatrixMinBits the set-up of a number on a whole wavefront costs more than
 // its squarings save.  A caller that forces a radix, lanes or an occupancy
 // keeps the lane kernels.
-constexpr uint32_t kMatrixCycles[6] = {0, 420, 550, 735, 825, 1150};  // by container
+constexpr uint32_t kMatrixCycles[6] = {0, 400, 480, 590, 710, 1110};  // by container
 
 uint32_t pgap_engine::matrix_limit(int digits, int blocks) const {
     const uint64_t L = (uint64_t)digits, simds = 4ull * (uint64_t)num_cus;

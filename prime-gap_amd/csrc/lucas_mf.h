@@ -115,20 +115,19 @@ __device__ __forceinline__ void lucas_step(const Wave<KB> &wx, const Wave<KB> &w
     v4i hx[T], hy[T], lx[T], ly[T];
     uint32_t p[T], r[T];
     int64_t s[T];
-#pragma unroll
-    for (int q = 0; q < T; ++q) hx[q] = hy[q] = v4i{0, 0, 0, 0};
     {
-        v4i a[KB + 3], bx[KB + 1], by[KB + 1];
+        v4i a[W::NA], bx[W::NB], by[W::NB], hbx[W::NBH], hby[W::NBH];
         wx.load_a_all(a);
         wx.load_b_low(bx);
         W::mul_low(lx, a, bx);
         wy.load_b_low(by);
         W::mul_low(ly, a, by);
-        v4i hbx[KB], hby[KB];
-        wx.load_b_high(hbx);
-        wy.load_b_high(hby);
-        W::template mul_high<3, KB + 3>(hx, a, hbx);
-        W::template mul_high<3, KB + 3>(hy, a, hby);
+        if constexpr (!W::L::shared) {
+            wx.load_b_high(hbx);
+            wy.load_b_high(hby);
+        }
+        W::high_of(hx, lx, a, bx, hbx);
+        W::high_of(hy, ly, a, by, hby);
     }
     wx.columns(lx, Weights(1), wx.k_low(BIAS), W::k_rest(BIAS), s);
     wx.carry(s, p);
@@ -137,7 +136,7 @@ __device__ __forceinline__ void lucas_step(const Wave<KB> &wx, const Wave<KB> &w
     wx.store_low(p);
     wy.store_low(r);
     {
-        v4i bx[KB + 1], by[KB + 1];
+        v4i bx[W::NB], by[W::NB];
         wx.load_b_low(bx);
         W::mul_low(lx, wx.ni, bx);
         wy.load_b_low(by);
@@ -150,19 +149,19 @@ __device__ __forceinline__ void lucas_step(const Wave<KB> &wx, const Wave<KB> &w
     wx.store_low(p);
     wy.store_low(r);
     {
-        v4i bx[KB], by[KB];
+        v4i bx[W::NBH], by[W::NBH];
         wx.load_b_high(bx);
-        W::template mul_high<0, KB>(hx, wx.nf, bx);
+        W::mul_high(hx, wx.nf, bx);
         wy.load_b_high(by);
-        W::template mul_high<0, KB>(hy, wx.nf, by);
+        W::mul_high(hy, wx.nf, by);
     }
     const Weights one(1);
 #pragma unroll
     for (int q = 0; q < T; ++q) s[q] = W::column(hx[q], one, c2[q]);
-    wx.carry(s, p);
+    wx.template carry<W::G0>(s, p);
 #pragma unroll
     for (int q = 0; q < T; ++q) s[q] = W::column(hy[q], one, cp[q]);
-    wx.carry(s, r);
+    wx.template carry<W::G0>(s, r);
     wx.store_high(p);
     wy.store_high(r);
 }
@@ -192,8 +191,8 @@ __device__ __forceinline__ uint32_t strong_lucas(const uint32_t *__restrict__ nw
     w.scale(n, b, 2, p);  // V'_0 = 2
 #pragma unroll
     for (int q = 0; q < T; ++q) {
-        const int i = 64 * q + (int)lane - 1;
-        c2[q] = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 ? value(w.buf[i]) : 0);
+        const int i = w.high_word(q);
+        c2[q] = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 && i < LW ? value(w.buf[i]) : 0);
     }
     // 1 / |Q|: (R mod N + k N) / |Q| with k making the division exact
     if (qa > 1) {
@@ -225,8 +224,8 @@ __device__ __forceinline__ uint32_t strong_lucas(const uint32_t *__restrict__ nw
     w.scale(n, b, 1, v1);
 #pragma unroll
     for (int q = 0; q < T; ++q) {
-        const int i = 64 * q + (int)lane - 1;
-        cp[q] = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 ? value(w.buf[i]) : 0);
+        const int i = w.high_word(q);
+        cp[q] = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 && i < LW ? value(w.buf[i]) : 0);
     }
 
     // (V'_j, V'_{j+1}) from j = 0 over the bits of m = N >> (tz + 1): X is the

@@ -2,7 +2,7 @@
 // wavefront: numbers are byte strings, and the three products of a Montgomery
 // squaring are convolutions of bytes that v_mfma_i32_16x16x64_i8 sums exactly.
 //
-// Representation.  x is LW = 16 KB - 1 words of four balanced bytes (digits in
+// Representation.  x is LW words (16 KB - 1 or 16 KB + 1) of four balanced bytes (digits in
 // [-128, 127], the operand type of the instruction), 4 LW digits of base 256;
 // R = 2^(32 LW).  A word of balanced bytes p has the value (p ^ 0x80808080) -
 // 0x80808080, so adding 0x80808080 to every word of a column sum, carrying
@@ -18,17 +18,22 @@
 // the accumulator layout (lane holds column lane % 16 and rows 4 (lane / 16) +
 // 0..3) lane l holds the four bytes of word base + l: words stay in lane order.
 // t runs in blocks of 64 (one instruction): block c starts at word 16 c - 15
-// for the tiles of the low half (bases 0, 64, ...) and 16 c - 1 for those of the
-// high half (bases LW - 1, LW + 63, ...).  LW = 15 mod 16 makes the A
-// fragments of both the same family, words 15 + 16 u + 16 (row / 4) - 4 (lane
+// for the tiles of the low half (bases 0, 64, ...) and 16 c + HOFF for those of
+// the high half (bases HB, HB + 64, ...).  With HB = HOFF + 15 mod 16 the A
+// fragments of both are one family, words 15 + 16 u + 16 (row / 4) - 4 (lane
 // / 16) downwards: A for block c of low tile q is fragment u = 4 q - c, of high
-// tile q it is u = KB - 1 + 4 q - c.  N (high tiles) and N^-1 mod R (low tiles)
+// tile q it is u = UH + 4 q - c.  N (high tiles) and N^-1 mod R (low tiles)
 // stay in registers as A fragments; B is read from the wave's LDS buffer.
+// Two layouts: HB = LW - 1 and HOFF = -1, the fewest instructions for LW = 15
+// mod 16; or HB a multiple of 16 and HOFF = -15, whose high tiles read the B
+// fragments of the low ones, and where HB is a multiple of 64 its first high
+// tile is the last low tile of the same product.  Layout gives each width the
+// one measured faster.
 //
 // Reduction.  T = a b; q = -T N^-1 mod R from the low tiles; (T + q N) / R from
-// the high tiles alone: they start one word below R, and everything beneath
-// that word adds less than 2^24 units of it, so rounding there is exact.  The high
-// columns of T are never carried: q N accumulates onto them.
+// the high tiles alone: everything beneath the word below R, word LW - 1, adds
+// less than 2^24 units of it, so rounding there is exact.  The high columns of T
+// are never carried: q N accumulates onto them.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -40,7 +45,18 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v4iu __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr uint32_t FLIP = 0x80808080u;
-constexpr int words(int KB) { return 16 * KB - 1; }
+// HB and HOFF of a width, see above.  Measured with both layouts, tests/s: 1108
+// bits (3 blocks) 3.67 -> 3.89 M with shared B fragments, 4247 (9) 232 -> 241 k;
+// 2128 (5) the same, where LW - 1 has the lower latency.
+constexpr bool shared_layout(int KB) { return KB == 3 || KB == 9; }
+template <int KB>
+struct Layout {
+    static constexpr bool shared = shared_layout(KB);
+    static constexpr int LW = shared ? 16 * KB + 1 : 16 * KB - 1;
+    static constexpr int HB = shared ? (KB < 4 ? 16 * KB : KB / 4 * 64) : LW - 1;
+    static constexpr int HOFF = shared ? -15 : -1;
+};
+constexpr int words(int KB) { return shared_layout(KB) ? 16 * KB + 1 : 16 * KB - 1; }
 // Bits a width takes: 16 below R for the lazy bounds (bases up to 63).
 constexpr int max_bits(int KB) { return 32 * words(KB) - 16; }
 
@@ -84,13 +100,22 @@ constexpr uint32_t BIAS_DIV = 1u << 24;   // words plus a multiple below 2^23 of
 
 template <int KB>
 struct Wave {
-    static constexpr int LW = words(KB), T = (KB + 3) / 4;
+    typedef Layout<KB> L;
+    static constexpr int LW = L::LW, HB = L::HB;
+    static constexpr int T = (LW + 63) / 64;                   // low tiles, and high ones
+    static constexpr int UMAX = LW / 16, NA = UMAX + 4;        // A fragments u = -3 .. UMAX
+    static constexpr int UH = (HB - L::HOFF - 15) / 16;
+    static constexpr int NB = (LW + 14) / 16 + 1;              // B blocks of the low tiles
+    static constexpr int NBH = (LW - 1 - L::HOFF) / 16 + 1;    // ... of the high ones
+    static constexpr int G0 = LW - 1 - HB;                     // lane of word LW - 1 in the first high tile
+    static_assert((2 * LW - HB + 63) / 64 == T, "as many high tiles as low ones");
+    static_assert((HB - L::HOFF) % 16 == 15 && 15 + 16 * (UMAX / 4 * 4) + 48 < 16 * KB + 60, "fragments");
     uint32_t *buf;                // word 0 of the wave's operand
     const uint32_t *pa, *pb;      // this lane's A and B fragment origins
     uint32_t *st_lo, *st_hi0, *st_hi;  // store addresses of the last low tile, the first and last high tile
     uint32_t sel, lane;
-    v4i nf[KB];      // N as A fragments u = 0 .. KB - 1
-    v4i ni[KB + 3];  // N^-1 mod R, u = -3 .. KB - 1
+    v4i nf[NA];  // N as A fragments (those the high tiles use)
+    v4i ni[NA];  // N^-1 mod R (the low tiles)
 
     __device__ __forceinline__ void init(uint32_t *lds, uint32_t l) {
         attach(lds, l);
@@ -107,8 +132,9 @@ struct Wave {
         uint32_t *dummy = buf + 16 * KB + 60;
         const int last = 64 * (T - 1);
         st_lo = (int)l + last < LW ? buf + l + last : dummy;
-        st_hi = (int)l + last >= 1 && (int)l + last <= LW ? buf + l + last - 1 : dummy;
-        st_hi0 = l >= 1 ? buf + l - 1 : dummy;
+        const int hi = (int)l + last - G0 - 1, hi0 = (int)l - G0 - 1;
+        st_hi = hi >= 0 && hi < LW ? buf + hi : dummy;
+        st_hi0 = hi0 >= 0 ? buf + hi0 : dummy;
     }
 
     // A fragment u of the number in the buffer.
@@ -123,18 +149,18 @@ struct Wave {
         return f;
     }
     // Lane 16 h + 4 g + j of fragment u holds piece u + g of the number (16
-    // words; pieces outside 0 .. KB - 1 are zero), so one load in four is
+    // words; pieces outside 0 .. UMAX are zero), so one load in four is
     // enough: the fragments between are its rows moved by 4 lanes a step, at
     // 1 or 2 moves a word against 1.2 words loaded and a permute.  The
     // kernel is bound by LDS reads (a squaring read 159 cycles of them at 1108
     // bits, 109 now) as much as by the vector ALU: 3.06 -> 3.90 M tests/s at 1108
     // bits, 1.0 -> 1.07 at 2128, 237 -> 248 k at 4247.  Moving words for the B
     // fragments too (2 moves each) costs more than the reads they replace.
-    __device__ __forceinline__ void load_a_all(v4i (&a)[KB + 3]) const {
+    __device__ __forceinline__ void load_a_all(v4i (&a)[NA]) const {
 #pragma unroll
-        for (int b = 0; b < KB; b += 4) a[b + 3] = load_a(b);
+        for (int b = 0; b <= UMAX; b += 4) a[b + 3] = load_a(b);
 #pragma unroll
-        for (int u = -3; u < KB; ++u) {
+        for (int u = -3; u <= UMAX; ++u) {
             if (u >= 0 && u % 4 == 0) continue;
             const v4i z = {0, 0, 0, 0};
             if (u < 0) {
@@ -142,7 +168,7 @@ struct Wave {
             } else {
                 const int b = u / 4 * 4, r = u % 4;
                 v4i up = z;
-                if (b + 4 < KB) {
+                if (b + 4 <= UMAX) {
                     const v4i &f = a[b + 7];
                     up = r == 1 ? shift<0x11C>(z, f) : r == 2 ? shift<0x118>(z, f) : shift<0x114>(z, f);
                 }
@@ -165,53 +191,70 @@ struct Wave {
     // The barrier keeps the loads together: left to itself the compiler loads
     // two blocks at a time and the matrix core idles for an LDS latency
     // between them.
-    __device__ __forceinline__ void load_b_low(v4i (&b)[KB + 1]) const {
+    __device__ __forceinline__ void load_b_low(v4i (&b)[NB]) const {
 #pragma unroll
-        for (int c = 0; c <= KB; ++c) b[c] = *(const v4iu *)(pb + 16 * c - 15);
+        for (int c = 0; c < NB; ++c) b[c] = *(const v4iu *)(pb + 16 * c - 15);
         __builtin_amdgcn_sched_barrier(0);
     }
-    __device__ __forceinline__ void load_b_high(v4i (&b)[KB]) const {
+    __device__ __forceinline__ void load_b_high(v4i (&b)[NBH]) const {
 #pragma unroll
-        for (int c = 0; c < KB; ++c) b[c] = *(const v4iu *)(pb + 16 * c - 1);
+        for (int c = 0; c < NBH; ++c) b[c] = *(const v4iu *)(pb + 16 * c + L::HOFF);
         __builtin_amdgcn_sched_barrier(0);
     }
 
     // Low tiles of A times B (columns of words 0 ..).
-    __device__ __forceinline__ static void mul_low(v4i (&acc)[T], const v4i (&a)[KB + 3], const v4i (&b)[KB + 1]) {
+    __device__ __forceinline__ static void mul_low(v4i (&acc)[T], const v4i (&a)[NA], const v4i (&b)[NB]) {
 #pragma unroll
         for (int q = 0; q < T; ++q) acc[q] = v4i{0, 0, 0, 0};
 #pragma unroll
-        for (int c = 0; c <= KB; ++c)
+        for (int c = 0; c < NB; ++c)
 #pragma unroll
             for (int q = 0; q < T; ++q)
-                if (c <= 4 * q + 3)
+                if (4 * q - c >= -3 && 4 * q - c <= UMAX)
                     acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[4 * q - c + 3], b[c], acc[q], 0, 0, 0);
     }
-    // High tiles (columns of words LW - 1 ..), added to acc; a[u + OFF] is
-    // fragment u.
-    template <int OFF, int NA>
-    __device__ __forceinline__ static void mul_high(v4i (&acc)[T], const v4i (&a)[NA], const v4i (&b)[KB]) {
+    // High tiles q0 .. (columns of words HB + 64 q ..), added to acc.
+    __device__ __forceinline__ static void mul_high(v4i (&acc)[T], const v4i (&a)[NA], const v4i (&b)[NBH],
+                                                    int q0 = 0) {
 #pragma unroll
-        for (int c = 0; c < KB; ++c)
+        for (int c = 0; c < NBH; ++c)
 #pragma unroll
             for (int q = 0; q < T; ++q)
-                if (c >= 4 * q)
-                    acc[q] =
-                        __builtin_amdgcn_mfma_i32_16x16x64_i8(a[KB - 1 + 4 * q - c + OFF], b[c], acc[q], 0, 0, 0);
+                if (q >= q0 && UH + 4 * q - c >= -3 && UH + 4 * q - c <= UMAX)
+                    acc[q] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[UH + 4 * q - c + 3], b[c], acc[q], 0, 0, 0);
+    }
+    // The high tiles of a product whose low tiles are lo and low B fragments bl.
+    __device__ __forceinline__ static void high_of(v4i (&hi)[T], const v4i (&lo)[T], const v4i (&a)[NA],
+                                                   const v4i (&bl)[NB], const v4i (&bh)[NBH]) {
+#pragma unroll
+        for (int q = 0; q < T; ++q) hi[q] = v4i{0, 0, 0, 0};
+        if constexpr (L::shared) {
+            if constexpr (HB % 64 == 0) {
+                hi[0] = lo[HB / 64];
+                mul_high(hi, a, bl, 1);
+            } else {
+                mul_high(hi, a, bl);
+            }
+        } else {
+            mul_high(hi, a, bh);
+        }
     }
 
     // Base-2^32 carries over the T x 64 words of s (every true carry plus the
     // bias is non-negative), then balanced bytes.
+    // G: the lowest word's lane (lanes below it hold nothing).
+    template <int G = 0>
     __device__ __forceinline__ void carry(const int64_t (&s)[T], uint32_t (&p)[T]) const {
         uint32_t prev = 0;
         uint64_t cy[T], any = 0;
 #pragma unroll
         for (int q = 0; q < T; ++q) {
             const uint32_t rot = wave_ror((uint32_t)((uint64_t)s[q] >> 32));
-            const uint32_t in = lane == 0 ? prev : rot;
+            const uint32_t in = lane <= (q == 0 ? G : 0) ? prev : rot;
             prev = rot;
             p[q] = (uint32_t)s[q] + in;
             cy[q] = __ballot(p[q] < in);
+            if (q == 0) cy[q] &= ~0ull << G;
             any |= cy[q];
         }
         // a carry out of a word is rare: its addend is below 2^19 (2^25 with
@@ -226,6 +269,7 @@ struct Wave {
                 const uint32_t one = (uint32_t)(in >> lane) & 1u;
                 p[q] += one;
                 cy[q] = __ballot(p[q] < one);
+                if (q == 0) cy[q] &= ~0ull << G;
                 any |= cy[q];
             }
         }
@@ -242,7 +286,7 @@ struct Wave {
         return lane == 0 ? ((int64_t)bias << 32) + FLIP : k_rest(bias);
     }
     __device__ __forceinline__ int64_t k_high(uint32_t bias) const {
-        return lane == 0 ? ((int64_t)bias << 32) + 0x80000000u : k_rest(bias);
+        return lane == G0 ? ((int64_t)bias << 32) + 0x80000000u : k_rest(bias);
     }
     __device__ __forceinline__ static int64_t column(const v4i &a, const Weights &w, int64_t k) {
         return k + (int64_t)a.x * w.w0 + (int64_t)a.y * w.w1 + (int64_t)a.z * w.w2 + (int64_t)a.w * w.w3;
@@ -253,8 +297,11 @@ struct Wave {
         for (int q = 0; q < T; ++q) s[q] = column(acc[q], w, q == 0 ? k0 : k);
     }
 
+    // The number's word that lane l of high tile q holds.
+    __device__ __forceinline__ int high_word(int q) const { return 64 * q + (int)lane - G0 - 1; }
+
     // Balanced words into the buffer: low tiles hold words 0 .., high tiles
-    // words -1 ...
+    // high_word().
     __device__ __forceinline__ void store_low(const uint32_t (&p)[T]) const {
         lds_order();
 #pragma unroll
@@ -265,7 +312,7 @@ struct Wave {
     __device__ __forceinline__ void store_high(const uint32_t (&p)[T]) const {
         lds_order();
 #pragma unroll
-        for (int q = 0; q < T - 1; ++q) *(q == 0 ? st_hi0 : buf + 64 * q + lane - 1) = p[q];
+        for (int q = 0; q < T - 1; ++q) *(q == 0 ? st_hi0 : buf + high_word(q)) = p[q];
         *st_hi = p[T - 1];
         lds_order();
     }
@@ -276,7 +323,7 @@ struct Wave {
         v4i acc[T];
         int64_t s[T];
         uint32_t p[T];
-        v4i b[KB + 1];
+        v4i b[NB];
         load_b_low(b);
         mul_low(acc, ni, b);
         columns(acc, Weights(-1), k_low(BIAS), k_rest(BIAS), s);
@@ -286,16 +333,14 @@ struct Wave {
 
     // buffer <- buffer^2 R^-1 mult mod N; p: the result's words (high layout).
     __device__ __forceinline__ void square(int32_t mult, uint32_t bias, uint32_t (&p)[T]) const {
-        v4i hi[T], lo[T], bh[KB], bl[KB + 1], a[KB + 3];
+        v4i hi[T], lo[T], bh[NBH], bl[NB], a[NA];
         int64_t s[T];
-#pragma unroll
-        for (int q = 0; q < T; ++q) hi[q] = v4i{0, 0, 0, 0};
         load_a_all(a);
-        load_b_high(bh);
+        if constexpr (!L::shared) load_b_high(bh);
         load_b_low(bl);
         mul_low(lo, a, bl);
         // the high columns of T are summed while its low words are carried
-        mul_high<3, KB + 3>(hi, a, bh);
+        high_of(hi, lo, a, bl, bh);
         columns(lo, Weights(1), k_low(BIAS), k_rest(BIAS), s);
         carry(s, p);
         store_low(p);
@@ -306,9 +351,9 @@ struct Wave {
         carry(s, p);
         store_low(p);
         load_b_high(bh);
-        mul_high<0, KB>(hi, nf, bh);
+        mul_high(hi, nf, bh);
         columns(hi, Weights(mult), k_high(bias), k_rest(bias), s);
-        carry(s, p);
+        carry<G0>(s, p);
         store_high(p);
     }
 
@@ -323,19 +368,19 @@ struct Wave {
         quotient();
 #pragma unroll
         for (int q = 0; q < T; ++q) hi[q] = v4i{0, 0, 0, 0};
-        v4i b[KB];
+        v4i b[NBH];
         load_b_high(b);
-        mul_high<0, KB>(hi, nf, b);
+        mul_high(hi, nf, b);
         columns(hi, Weights(1), k_high(BIAS), k_rest(BIAS), s);
-        carry(s, p);
+        carry<G0>(s, p);
         bool rest = false;  // some word above the lowest is not zero
 #pragma unroll
         for (int q = 0; q < T; ++q) {
-            const int w = 64 * q + (int)lane - 1;
+            const int w = high_word(q);
             rest |= w >= 1 && w < LW && p[q] != 0;
         }
         if (__ballot(rest) != 0) return 0;
-        const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)p[0], 1);
+        const uint32_t w0 = (uint32_t)__builtin_amdgcn_readlane((int)p[0], G0 + 1);
         return w0 == 1u ? 1u : (w0 == 0xffu ? 2u : (w0 == 0u ? 3u : 0u));
     }
 
@@ -350,7 +395,7 @@ struct Wave {
         store_low(p);
         load_a_all(ni);  // N for now
 #pragma unroll
-        for (int u = 0; u < KB; ++u) nf[u] = ni[u + 3];
+        for (int u = 0; u < NA; ++u) nf[u] = ni[u];
         // N^-1 by Newton's iteration y <- y (2 - N y), 30 bits to start
         const uint32_t n0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)n[0]);
         uint32_t y0 = n0;
@@ -361,7 +406,7 @@ struct Wave {
         store_low(p);
 #pragma unroll 1
         for (int prec = 30; prec < 32 * LW; prec *= 2) {
-            v4i y[KB + 3], bl[KB + 1], acc[T];
+            v4i y[NA], bl[NB], acc[T];
             load_a_all(y);
             load_b_low(bl);
             mul_low(acc, ni, bl);

@@ -23,11 +23,11 @@ def check(engine, vals, kind, bases=(), limbs=None):
     return got
 
 
-# containers of 15, 31, ... 143 words take 32 words - 16 bits
-@pytest.mark.parametrize("blocks", range(1, 10))
-def test_container_edges(engine, blocks):
-    top = min(32 * (16 * blocks - 1) - 16, 4466)  # the widest that every base takes
-    rng = random.Random(blocks)
+# containers of 16 k - 1 words (15, 31, 63, ...) or 16 k + 1 (49, 145) take 32
+# words - 16 bits; 4466 is the widest that every base takes
+@pytest.mark.parametrize("top", [464, 976, 1488, 1552, 2000, 2512, 3024, 3536, 4048, 4466])
+def test_container_edges(engine, top):
+    rng = random.Random(top)
     vals = [(1 << top) - 1, (1 << top) - 3, (1 << (top - 1)) + 1, (1 << top) - (1 << (top // 2)) - 1]
     vals += [rng.getrandbits(b) | (1 << (b - 1)) | 1 for b in (top, top, top - 1, top - 15, top - 16, top - 31, 257)]
     # every word of the quotient at the ends of the balanced range
@@ -61,12 +61,11 @@ def test_remainder_of_a_round(engine, kind, bases):
         assert engine.last_launch().matrix_tests == (count - 65536 if count - 65536 <= 1000 else 0)
 
 
-@pytest.mark.parametrize("blocks", range(1, 10))
-def test_strong_lucas_edges(engine, blocks):
+@pytest.mark.parametrize("top", [464, 976, 1488, 1552, 2000, 2512, 3024, 3536, 4048, 4472])
+def test_strong_lucas_edges(engine, top):
     # the Lucas chain's set-up (parameter search, 1 / Q, N = 2^b - 1) and its
     # width bounds, against the oracle and the lane variant's bound of 4472
-    top = min(32 * (16 * blocks - 1) - 16, 4472)
-    rng = random.Random(100 + blocks)
+    rng = random.Random(100 + top)
     vals = list(range(0, 130)) + [5459, 5777, 10877, 16109, 18971, 1093 ** 2, 3511 ** 2, (1 << 61) - 1]
     vals += [(1 << top) - 1, (1 << top) - 3, (1 << (top - 1)) + 1, (rng.getrandbits(top // 2) | 1) ** 2]
     vals += [rng.getrandbits(b) | (1 << (b - 1)) | 1 for b in (top, top, top - 15, top - 31)]
@@ -94,7 +93,7 @@ def test_mixed_batch_on_both_kernels(engine, kind, bases):
     rng = random.Random(7)
     vals = [rng.getrandbits(300) | (1 << 299) | 1 for _ in range(5000)]
     vals += [rng.getrandbits(b) | (1 << (b - 1)) | 1 for b in (700, 720, 1100, 2100, 2180, 2250, 4400)]
-    vals += [rng.getrandbits(32 * (16 * k - 1) - 16) | 1 for k in range(1, 9)]
+    vals += [rng.getrandbits(32 * (16 * k - 1) - 16) | 1 for k in range(1, 9)] + [rng.getrandbits(b) | 1 for b in (1489, 1552, 1553)]
     vals += [(1 << p) - 1 for p in MERSENNE] + [3 * ((1 << p) - 1) for p in MERSENNE] + [0, 1, 2, 3, 5, 2047, 341]
     rng.shuffle(vals)
     got = engine.prp_mixed([pgap.to_limbs([v], pgap.limbs_needed(v))[0] for v in vals], kind, bases)
