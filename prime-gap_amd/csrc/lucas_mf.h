@@ -1,5 +1,5 @@
 // lucas_mf.h -- strong Lucas probable-prime test (Selfridge's method A) of one
-// number per wavefront on the matrix cores (mont_mf.h).  The verdict is
+// number per workgroup on the matrix cores (mont_mf.h).  The verdict is
 // lucas_lg.h's: U_d = 0 or V_{d 2^r} = 0 (mod N) for some 0 <= r < s, with
 // N + 1 = d 2^s, P = 1, Q = (1 - D) / 4.
 //
@@ -12,11 +12,16 @@
 //     V_d = V_{d+1} + Q V_{d-1} = Q^(m+1) (V'_{m+1} + V'_m),
 //   V_{d 2^r} = Q^(d 2^(r-1)) V'_{d 2^(r-1)} for r > 0, V'_d = V'_m V'_{m+1} - P'.
 //
-// The two products of a step are independent and run interleaved: a step
-// takes twice a squaring's matrix instructions, 3.3 thousand cycles at 2128
-// bits (2.9 ms a test, 3.2 ms for 1024, 13.8 ms for 8192) against 11.9 thousand
-// for the row-wise products of lucas_wave_kernel (10.3 ms) and 47 thousand on
-// 8 lanes (41.7 ms, 49 ms for 8192).
+// The two products of a step are independent: two wavefronts of a workgroup take
+// one each and trade the results through LDS, one barrier a step, so a step has
+// a squaring's latency, which is what few numbers are bound by (a scan's round
+// lasts as long as its Lucas tests).  Both do the set-up and the final tests
+// alike.  One wavefront per number against two, ms for 64 / 1024 / 16384
+// numbers: 1108 bits 0.95 / 1.03 / 6.4 -> 0.65 / 0.85 / 7.3, 2128 bits 2.76 / 2.97 /
+// 23.9 -> 1.83 / 2.54 / 28.3, 4247 bits 9.7 / 10.2 / 122 -> 6.1 / 8.6 / 98 (there
+// both products' fragments spilled).  Filled up it is bound by LDS reads like a
+// squaring and the A fragments are loaded by both, the 13 to 18% above; numbers
+// that get this far are few, so there is no second form for that.
 #pragma once
 #include "lucas_lg.h"
 #include "prp_mf.h"
@@ -105,73 +110,50 @@ __device__ __forceinline__ int32_t selfridge(const uint32_t *__restrict__ nw, ui
     return 0;
 }
 
-// X^2 R^-1 - c2 into X's buffer and X Y R^-1 - cp into Y's, as balanced words
-// (c2, cp: the high tiles' per-word constants with the subtrahend taken off).
+// LDS of a test: (V'_j, V'_{j+1}) twice, for reading and writing, and a work
+// buffer per wavefront.
+constexpr int lucas_words(int KB) { return 6 * buf_words(KB); }
+
+// x y R^-1 - c into out's buffer (c: the high tiles' per-word constants with
+// the subtrahend taken off); w's buffer is overwritten.
 template <int KB>
-__device__ __forceinline__ void lucas_step(const Wave<KB> &wx, const Wave<KB> &wy, const int64_t (&c2)[Wave<KB>::T],
-                                           const int64_t (&cp)[Wave<KB>::T]) {
+__device__ __forceinline__ void lucas_product(const Wave<KB> &w, const Wave<KB> &x, const Wave<KB> &y,
+                                              const Wave<KB> &out, const int64_t (&c)[Wave<KB>::T]) {
     typedef Wave<KB> W;
     constexpr int T = W::T;
-    v4i hx[T], hy[T], lx[T], ly[T];
-    uint32_t p[T], r[T];
+    v4i hi[T], lo[T], a[W::NA], bl[W::NB], bh[W::NBH];
+    uint32_t p[T];
     int64_t s[T];
-    {
-        v4i a[W::NA], bx[W::NB], by[W::NB], hbx[W::NBH], hby[W::NBH];
-        wx.load_a_all(a);
-        wx.load_b_low(bx);
-        W::mul_low(lx, a, bx);
-        wy.load_b_low(by);
-        W::mul_low(ly, a, by);
-        if constexpr (!W::L::shared) {
-            wx.load_b_high(hbx);
-            wy.load_b_high(hby);
-        }
-        W::high_of(hx, lx, a, bx, hbx);
-        W::high_of(hy, ly, a, by, hby);
-    }
-    wx.columns(lx, Weights(1), wx.k_low(BIAS), W::k_rest(BIAS), s);
-    wx.carry(s, p);
-    wx.columns(ly, Weights(1), wx.k_low(BIAS), W::k_rest(BIAS), s);
-    wx.carry(s, r);
-    wx.store_low(p);
-    wy.store_low(r);
-    {
-        v4i bx[W::NB], by[W::NB];
-        wx.load_b_low(bx);
-        W::mul_low(lx, wx.ni, bx);
-        wy.load_b_low(by);
-        W::mul_low(ly, wx.ni, by);
-    }
-    wx.columns(lx, Weights(-1), wx.k_low(BIAS), W::k_rest(BIAS), s);
-    wx.carry(s, p);
-    wx.columns(ly, Weights(-1), wx.k_low(BIAS), W::k_rest(BIAS), s);
-    wx.carry(s, r);
-    wx.store_low(p);
-    wy.store_low(r);
-    {
-        v4i bx[W::NBH], by[W::NBH];
-        wx.load_b_high(bx);
-        W::mul_high(hx, wx.nf, bx);
-        wy.load_b_high(by);
-        W::mul_high(hy, wx.nf, by);
-    }
+    x.load_a_all(a);
+    if constexpr (!W::L::shared) y.load_b_high(bh);
+    y.load_b_low(bl);
+    W::mul_low(lo, a, bl);
+    W::high_of(hi, lo, a, bl, bh);
+    w.columns(lo, Weights(1), w.k_low(BIAS), W::k_rest(BIAS), s);
+    w.carry(s, p);
+    w.store_low(p);
+    w.load_b_low(bl);
+    W::mul_low(lo, w.ni, bl);
+    w.columns(lo, Weights(-1), w.k_low(BIAS), W::k_rest(BIAS), s);
+    w.carry(s, p);
+    w.store_low(p);
+    w.load_b_high(bh);
+    W::mul_high(hi, w.nf, bh);
     const Weights one(1);
 #pragma unroll
-    for (int q = 0; q < T; ++q) s[q] = W::column(hx[q], one, c2[q]);
-    wx.template carry<W::G0>(s, p);
-#pragma unroll
-    for (int q = 0; q < T; ++q) s[q] = W::column(hy[q], one, cp[q]);
-    wx.template carry<W::G0>(s, r);
-    wx.store_high(p);
-    wy.store_high(r);
+    for (int q = 0; q < T; ++q) s[q] = W::column(hi[q], one, c[q]);
+    w.template carry<W::G0>(s, p);
+    out.store_high(p);
 }
 
+// A test by a workgroup of two wavefronts (`wave` 0 and 1), every thread in it.
 template <int KB>
 __device__ __forceinline__ uint32_t strong_lucas(const uint32_t *__restrict__ nw, uint32_t limbs, uint32_t *lds,
-                                                 uint32_t lane) {
+                                                 uint32_t wave, uint32_t lane) {
     typedef Wave<KB> W;
     constexpr int T = W::T, LW = W::LW;
-    W w, wy;
+    constexpr int BW = buf_words(KB);
+    W w;
     uint32_t n[T], p[T], b;
     if (!load_n<KB>(nw, limbs, lane, n, &b)) return b == 2 && (nw[0] & 1u) == 0 ? 1u : 0u;  // 2 passes
     const int32_t D = selfridge<KB>(nw, limbs, b, lane);
@@ -181,10 +163,13 @@ __device__ __forceinline__ uint32_t strong_lucas(const uint32_t *__restrict__ nw
     const uint32_t ninv = qa > 1 ? inverse_small(lg::words_mod(nw, (b + 31) / 32, qa), qa) : 1u;
     if (ninv == 0) return 0;  // a prime divides Q and N
 
-    w.init(lds, lane);
-    wy.init(lds + buf_words(KB), lane);
+    // buffers 2 par + i: V'_{j+i}; 4 + wave: work
+    __syncthreads();  // the workgroup's previous test has been read
+    w.init(lds + wave * BW, lane);  // the wavefront's own V' is stored before the next barrier
+    w.init(lds + (2 + wave) * BW, lane);
+    w.init(lds + (4 + wave) * BW, lane);
     w.setup(n, b, p);  // R mod N
-    int64_t s[T], c2[T], cp[T];
+    int64_t s[T], c[T];
     uint32_t one[T];
 #pragma unroll
     for (int q = 0; q < T; ++q) one[q] = p[q];
@@ -192,7 +177,7 @@ __device__ __forceinline__ uint32_t strong_lucas(const uint32_t *__restrict__ nw
 #pragma unroll
     for (int q = 0; q < T; ++q) {
         const int i = w.high_word(q);
-        c2[q] = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 && i < LW ? value(w.buf[i]) : 0);
+        c[q] = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 && i < LW ? value(w.buf[i]) : 0);
     }
     // 1 / |Q|: (R mod N + k N) / |Q| with k making the division exact
     if (qa > 1) {
@@ -222,72 +207,67 @@ __device__ __forceinline__ uint32_t strong_lucas(const uint32_t *__restrict__ nw
     uint32_t v1[T];
     w.carry(s, v1);
     w.scale(n, b, 1, v1);
+    // what this wavefront subtracts: 2 from X^2, P' from X Y
 #pragma unroll
     for (int q = 0; q < T; ++q) {
         const int i = w.high_word(q);
-        cp[q] = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 && i < LW ? value(w.buf[i]) : 0);
+        const int64_t cp = (q == 0 ? w.k_high(BIAS) : W::k_rest(BIAS)) - (i >= 0 && i < LW ? value(w.buf[i]) : 0);
+        c[q] = wave ? cp : c[q];
     }
 
-    // (V'_j, V'_{j+1}) from j = 0 over the bits of m = N >> (tz + 1): X is the
-    // one the next bit squares
+    // (V'_j, V'_{j+1}) from j = 0 over the bits of m = N >> (tz + 1): X = V'_{j+bit}
     uint32_t tz = 0;  // N + 1 = d 2^tz
     while (tz < b && ((nw[tz >> 5] >> (tz & 31)) & 1u)) ++tz;
-    w.store_low(p);    // X's buffer: V'_0
-    wy.store_low(v1);  // Y's: V'_1
-    bool high = false;  // X's buffer holds V'_{j+1}
+    W x, y, out;
+    x.attach(lds + wave * BW, lane);
+    if (wave == 0)
+        x.store_low(p);  // V'_0
+    else
+        x.store_low(v1);  // V'_1
+    uint32_t par = 0;
+    const auto step = [&](uint32_t bit) {
+        __syncthreads();
+        x.attach(lds + (2 * par + bit) * BW, lane);
+        y.attach(lds + (2 * par + (wave ? 1 - bit : bit)) * BW, lane);
+        par ^= 1;
+        // X^2 - 2 is V'_{2j} (bit 0) or V'_{2j+2} (bit 1), X Y - P' is V'_{2j+1}
+        out.attach(lds + (2 * par + (wave ? 1 - bit : bit)) * BW, lane);
+        lucas_product<KB>(w, x, y, out, c);
+    };
 #pragma unroll 1
-    for (int i = (int)b - 1; i > (int)tz; --i) {
-        const bool bit = (nw[i >> 5] >> (i & 31)) & 1u;
-        if (bit != high) {  // square the other one
-            uint32_t *t = w.buf;
-            w.attach(wy.buf - PAD, lane);
-            wy.attach(t - PAD, lane);
-        }
-        lucas_step<KB>(w, wy, c2, cp);
-        // X^2 - 2 is V'_{2j} (bit 0) or V'_{2j+2} (bit 1)
-        high = bit;
-    }
-    // V'_{m+1} -+ V'_m, then the V'_{d 2^i}
-    uint32_t x[T], y[T];
-    lds_order();
+    for (int i = (int)b - 1; i > (int)tz; --i) step((nw[i >> 5] >> (i & 31)) & 1u);
+    __syncthreads();
+    // V'_{m+1} -+ V'_m
+    uint32_t v0[T];
+    const auto state = [&](uint32_t i, uint32_t (&v)[T]) {
+        const uint32_t *buf = lds + (2 * par + i) * BW + PAD;
 #pragma unroll
-    for (int q = 0; q < T; ++q) {
-        const int i = 64 * q + (int)lane;
-        x[q] = i < LW ? w.buf[i] : 0u;
-        y[q] = i < LW ? wy.buf[i] : 0u;
-    }
-    lds_order();
+        for (int q = 0; q < T; ++q) v[q] = 64 * q + (int)lane < LW ? buf[64 * q + lane] : 0u;
+    };
+    state(0, v0);
+    state(1, v1);
 #pragma unroll
     for (int sign = 0; sign < 2; ++sign) {
 #pragma unroll
         for (int q = 0; q < T; ++q)
-            s[q] = value(x[q]) + (sign ? value(y[q]) : -value(y[q])) + (q == 0 ? w.k_low(BIAS) : W::k_rest(BIAS));
+            s[q] = value(v1[q]) + (sign ? value(v0[q]) : -value(v0[q])) + (q == 0 ? w.k_low(BIAS) : W::k_rest(BIAS));
         w.carry(s, p);
         w.store_low(p);
         if (w.classify() == 3) return 1;
     }
     if (tz < 2) return 0;
-    // V'_d = V'_m V'_{m+1} - P' in Y's buffer
-    w.store_low(x);
-    wy.store_low(y);
-    lucas_step<KB>(w, wy, c2, cp);
+    // V'_d = V'_m V'_{m+1} - P' (bit 0 writes it as V'_{j+1}), then V'_2k = V'_k^2 -
+    // 2, wavefront 0's product with X = V'_k (bit 1 writes it as V'_{j+1} too)
+    step(0);
 #pragma unroll 1
-    for (uint32_t r = 1; r < tz; ++r) {
-        lds_order();
-#pragma unroll
-        for (int q = 0; q < T; ++q) {
-            const int i = 64 * q + (int)lane;
-            y[q] = i < LW ? wy.buf[i] : 0u;
-        }
-        lds_order();
-        w.store_low(y);
+    for (uint32_t r = 1;; ++r) {
+        __syncthreads();
+        state(1, v1);
+        w.store_low(v1);
         if (w.classify() == 3) return 1;
-        if (r + 1 == tz) break;
-        // V'_{2k} = V'_k^2 - 2: X = Y
-        w.store_low(y);
-        lucas_step<KB>(w, wy, c2, c2);
+        if (r + 1 >= tz) return 0;
+        step(1);
     }
-    return 0;
 }
 
 }  // namespace mf

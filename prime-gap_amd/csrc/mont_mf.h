@@ -93,7 +93,7 @@ struct Weights {
 };
 
 // Bias that keeps the carries out of words non-negative: above the largest
-// column sum's value over 2^32 (two products of 572 digits: 2^16.2 times mult).
+// column sum's value over 2^32 (two products of 580 digits: 2^16.2 times mult).
 constexpr uint32_t BIAS = 1u << 18;       // mult 1 or 2
 constexpr uint32_t BIAS_WIDE = 1u << 24;  // mult up to 63
 constexpr uint32_t BIAS_DIV = 1u << 24;   // words plus a multiple below 2^23 of words

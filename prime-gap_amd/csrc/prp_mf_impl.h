@@ -62,28 +62,29 @@ hipError_t launch_mf(const uint32_t *d_n, uint32_t limbs, uint32_t first, uint32
 // their own: with two engines in a process they shared one, and every round of
 // 1.9 to 5 ms (2128 bits) waited 2.75 ms for its Lucas batch.
 template <int KB>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
 scan_mf_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint32_t conf_rows, uint32_t conf_max,
                uint32_t max_items, const uint32_t *__restrict__ ctr, const uint8_t *__restrict__ base,
                uint8_t *__restrict__ out, const uint32_t *__restrict__ lnum, uint32_t nluc,
                uint8_t *__restrict__ lverd) {
-    __shared__ __align__(16) uint32_t lds[2 * mf::buf_words(KB)];
+    __shared__ __align__(16) uint32_t lds[mf::lucas_words(KB)];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
     const uint32_t nc = min(ctr[3], conf_max), nf = min(ctr[0], max_items);
+    // a Lucas test takes the workgroup, the others a wavefront each
+    uint32_t i = blockIdx.x;
 #pragma unroll 1
-    for (uint32_t i = blockIdx.x; i < nluc + nc + nf; i += gridDim.x) {
-        uint32_t v;
-        uint8_t *o;
-        if (i < nluc) {
-            v = mf::strong_lucas<KB>(lnum + (size_t)i * limbs, limbs, lds, threadIdx.x);
-            o = lverd + i;
-        } else {
-            const uint32_t r = i - nluc, row = r < nc ? r : conf_rows + (r - nc);
-            const uint32_t *nw = n + (size_t)row * limbs;
-            v = r < nc ? mf::sprp<KB>(nw, limbs, base[r], lds, threadIdx.x)
-                       : mf::fermat2<KB>(nw, limbs, lds, threadIdx.x);
-            o = out + row;
-        }
-        if (threadIdx.x == 0) *o = (uint8_t)v;
+    for (; i < nluc; i += gridDim.x) {
+        const uint32_t v = mf::strong_lucas<KB>(lnum + (size_t)i * limbs, limbs, lds, wave, lane);
+        if (threadIdx.x == 0) lverd[i] = (uint8_t)v;
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (uint32_t r = 2 * (i - nluc) + wave; r < nc + nf; r += 2 * gridDim.x) {
+        const uint32_t row = r < nc ? r : conf_rows + (r - nc);
+        const uint32_t *nw = n + (size_t)row * limbs;
+        uint32_t *buf = lds + wave * mf::buf_words(KB);
+        const uint32_t v = r < nc ? mf::sprp<KB>(nw, limbs, base[r], buf, lane) : mf::fermat2<KB>(nw, limbs, buf, lane);
+        if (lane == 0) out[row] = (uint8_t)v;
     }
 }
 
@@ -91,26 +92,26 @@ template <int KB>
 hipError_t launch_scan_mf(const uint32_t *d_n, uint32_t limbs, uint32_t conf_rows, uint32_t conf_max,
                           uint32_t max_items, const uint32_t *d_ctr, const uint8_t *d_base, uint8_t *d_out,
                           const uint32_t *d_lnum, uint32_t nluc, uint8_t *d_lverd, hipStream_t stream) {
-    const uint32_t blocks = std::min(nluc + conf_max + max_items, kMatrixBlocks);
+    const uint32_t blocks = std::min(nluc + (conf_max + max_items + 1) / 2, kMatrixBlocks / 2);
     if (blocks == 0) return hipSuccess;
-    hipLaunchKernelGGL((scan_mf_kernel<KB>), dim3(blocks), dim3(64), 0, stream, d_n, limbs, conf_rows, conf_max,
+    hipLaunchKernelGGL((scan_mf_kernel<KB>), dim3(blocks), dim3(128), 0, stream, d_n, limbs, conf_rows, conf_max,
                        max_items, d_ctr, d_base, d_out, d_lnum, nluc, d_lverd);
     return hipGetLastError();
 }
 
-// Strong Lucas: two products a step hold twice the fragments, so a wavefront
-// has the SIMD's registers to itself.
+// Strong Lucas: a workgroup of two wavefronts per number.
 template <int KB>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
 lucas_mf_kernel(const uint32_t *__restrict__ n, uint32_t limbs, uint32_t first, uint32_t count,
                 const uint32_t *__restrict__ d_first, const uint32_t *__restrict__ d_count,
                 const uint32_t *__restrict__ d_idx, uint8_t *__restrict__ out) {
-    __shared__ __align__(16) uint32_t lds[2 * mf::buf_words(KB)];
+    __shared__ __align__(16) uint32_t lds[mf::lucas_words(KB)];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
     const uint32_t cnt = d_count ? min(*d_count, count) : count;
 #pragma unroll 1
     for (uint32_t i = (d_first ? *d_first : first) + blockIdx.x; i < cnt; i += gridDim.x) {
         const uint32_t row = d_idx ? d_idx[i] : i;
-        const uint32_t v = mf::strong_lucas<KB>(n + (size_t)row * limbs, limbs, lds, threadIdx.x);
+        const uint32_t v = mf::strong_lucas<KB>(n + (size_t)row * limbs, limbs, lds, wave, lane);
         if (threadIdx.x == 0) out[row] = (uint8_t)v;
     }
 }
@@ -121,7 +122,7 @@ hipError_t launch_lucas_mf(const uint32_t *d_n, uint32_t limbs, uint32_t first, 
                            uint8_t *d_out, hipStream_t stream) {
     if (first >= count) return hipSuccess;
     const uint32_t blocks = d_count ? std::min(count, kMatrixBlocks) : count - first;
-    hipLaunchKernelGGL((lucas_mf_kernel<KB>), dim3(blocks), dim3(64), 0, stream, d_n, limbs, first, count, d_first,
+    hipLaunchKernelGGL((lucas_mf_kernel<KB>), dim3(blocks), dim3(128), 0, stream, d_n, limbs, first, count, d_first,
                        d_count, d_idx, d_out);
     return hipGetLastError();
 }
