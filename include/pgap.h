@@ -107,7 +107,7 @@ pgap_status pgap_prp_batch_device_noalloc(pgap_engine *e, uint32_t limbs, const 
                                           pgap_test kind, const uint32_t *bases, uint32_t nbases,
                                           uint8_t *d_verdict, uint32_t max_bits);
 
-/* Mixed widths in one persistent launch.  Number i has limbs[i] words
+/* Mixed widths in one call.  Number i has limbs[i] words
  * starting at words + offset[i].  Numbers are grouped into size buckets:
  * well-filled ones of up to 2180 bits run one lane per number from one work
  * queue, the others one number per wavefront on the matrix cores, up to 4476

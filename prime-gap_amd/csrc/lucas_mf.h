@@ -20,7 +20,7 @@
 // numbers: 1108 bits 0.95 / 1.03 / 6.4 -> 0.65 / 0.85 / 7.3, 2128 bits 2.76 / 2.97 /
 // 23.9 -> 1.83 / 2.54 / 28.3, 4247 bits 9.7 / 10.2 / 122 -> 6.1 / 8.6 / 98 (there
 // both products' fragments spilled).  Filled up it is bound by LDS reads like a
-// squaring and the A fragments are loaded by both, the 13 to 18% above; numbers
+// squaring and the A fragments are loaded by both, 15 to 25% below 3600 bits; numbers
 // that get this far are few, so there is no second form for that.
 #pragma once
 #include "lucas_lg.h"

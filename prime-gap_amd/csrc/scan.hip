@@ -19,9 +19,9 @@
 //   confirmation stage) -> per-slot update, emitting finished m's and
 //   exhausted sides.
 // Strong-PRP confirmations ride in the next round's grid instead of a launch
-// of their own, so a round costs one test's latency; strong Lucas rows (lane
-// groups only) run in a launch of their own on a second stream, beside the
-// grid, and are joined before the retire step.  A hit
+// of their own, so a round costs one test's latency; strong Lucas rows ride in
+// a grid of the matrix cores too, and beside a grid of the one-lane kernels
+// they run in a launch of their own on a second stream.  A hit
 // that fails a confirmation (a base-2 pseudoprime) restarts its side just
 // past it.
 // Every index below a side's first PRP has been tested in this or an earlier
@@ -67,6 +67,7 @@ constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may a
 constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
 constexpr uint32_t MATRIX_WAVES = 4;      // wavefronts per SIMD in a full matrix round
 constexpr uint32_t MATRIX_WAVES_HELD = 2;  // ... while few sides scan
+constexpr uint32_t LUCAS_LANES = 128;     // of a strong Lucas test on the matrix cores
 constexpr uint32_t LUCAS_POOLS = 4;  // Lucas batches that may run at once (a ring)
 
 enum : uint32_t {
@@ -208,8 +209,8 @@ __device__ __forceinline__ uint32_t side_weight(uint32_t cursor) { return 1u + m
 
 // ctr[1] = sides that run Fermat tests this round, ctr[4] = confirmation
 // rows, ctr[5] = the scanning sides' total weight, ctr[6] = confirming sides
-// (with Baillie-PSW, each starts a strong Lucas test that takes a whole
-// wavefront beside the grid; the Fermat rows divide the resident lanes the
+// (with Baillie-PSW, each starts a strong Lucas test of two wavefronts; the
+// Fermat rows divide the resident lanes the
 // confirmations leave among the scanning sides).
 __global__ void count_kernel(const uint32_t *__restrict__ active, uint32_t na, const SlotState *__restrict__ st,
                              uint32_t nconf, uint32_t *__restrict__ ctr) {
@@ -273,8 +274,8 @@ __global__ void issue_kernel(const uint32_t *__restrict__ active, uint32_t na, S
     const uint32_t c = s.cursor[side], l = s.len[side];
     const uint32_t ns = max(ctr[1], 1u), wsum = max(ctr[5], 1u), w = side_weight(c);
     // confirmation rows in whole wavefronts, and the lanes of the strong Lucas
-    // tests that run beside the grid (`lres` lanes each, in units of this
-    // grid's items of 64 / cpad lanes)
+    // tests (`lres` lanes each, in units of this grid's items of 64 / cpad
+    // lanes)
     const uint32_t used = (ctr[4] + cpad - 1) / cpad * cpad + (lpool ? (ctr[6] * lres * cpad + 63) / 64 : 0u);
     const uint32_t room = resident > used ? resident - used : 0u;
     // weighted shares, at least one item each: the sum stays within room
@@ -486,9 +487,8 @@ class Scanner {
     bool stop = false;
     std::thread worker;
     hipStream_t stream = nullptr;      // the worker's stream
-    // Strong Lucas confirmations (Baillie-PSW) are not part of a round's
-    // grid: a Lucas test costs more than a Fermat test, and a round is sized
-    // to one.  A round's Lucas tests (one per confirming side) go to a pool
+    // Strong Lucas confirmations (Baillie-PSW) are not part of a one-lane
+    // round's grid.  Such a round's Lucas tests (one per confirming side) go to a pool
     // of a ring of LUCAS_POOLS (the item and its number), which starts as a
     // batch right after the issue step on a stream of its own (default
     // priority; batches run there in order); finished batches are retired,
@@ -899,7 +899,7 @@ class Scanner {
 
     // Start pool p (n items, written by the issue step already queued on the
     // round's stream) as a batch on the Lucas stream.
-    // One number per wavefront on the matrix cores; a forced lane count keeps
+    // Two wavefronts per number on the matrix cores; a forced lane count keeps
     // that family's variant.
     pgap_status lucas_launch(uint32_t p, const Plan &c, uint32_t n) {
         Bases none{};
@@ -1046,10 +1046,10 @@ class Scanner {
                 return e->hip_fail(he, "scan count");
             nluc = h_ctr[6];
             if (nluc && mx) {
-                lres = 64;
+                lres = LUCAS_LANES;
             } else if (nluc) {
                 if ((st = e->plan(KIND_LUCAS, bits, none, &lc))) return st;
-                lres = resident < resident_full ? (lc.mx ? 64u : (uint32_t)lc.lane.v->lanes) : 0u;
+                lres = resident < resident_full ? (lc.mx ? LUCAS_LANES : (uint32_t)lc.lane.v->lanes) : 0u;
             }
         }
         hipLaunchKernelGGL(issue_kernel, dim3((2 * na + 255) / 256), b256, 0, stream, d_active, na, d_state, cr,
