@@ -198,7 +198,7 @@ class Engine:
     def __init__(self, device: int = 0, hbm_budget: int = 0, radix: int = 0, lanes: int = 0,
                  waves_per_simd: int = 0, tuning_path: Optional[str] = None):
         self.lib = load()
-        self._lists = None
+        self._lists = []
         opt = Options(device, hbm_budget, tuning_path.encode() if tuning_path else None, radix, lanes,
                       waves_per_simd)
         h = ctypes.c_void_p()
@@ -319,27 +319,31 @@ class Engine:
         """-> list of (prev distances, next distances) per m (device sieve)."""
         mm = np.ascontiguousarray(ms, dtype=np.uint64)
         n = len(mm)
-        prev, nxt = self._list_buffers(n, sieve_length)
+        buf = self._take_lists(2 * n * sieve_length)
+        prev, nxt = buf[:2 * n * sieve_length].reshape(2, n, sieve_length)
         npv = np.zeros(n, dtype=np.uint32)
         nnx = np.zeros(n, dtype=np.uint32)
         self._check(self.lib.pgap_sieve(self.h, family, mm.ctypes.data, n, max_prime, prev.ctypes.data,
                                         npv.ctypes.data, nxt.ctypes.data, nnx.ctypes.data))
-        return [(prev[i, : npv[i]].copy(), nxt[i, : nnx[i]].copy()) for i in range(n)]
+        lists = [(prev[i, : npv[i]].copy(), nxt[i, : nnx[i]].copy()) for i in range(n)]
+        if buf.nbytes <= self.LIST_BUFFER_BYTES and not self._lists:
+            self._lists.append(buf)
+        return lists
 
     # Bytes of list buffers an engine keeps between sieve calls.
     LIST_BUFFER_BYTES = 128 << 20
 
-    def _list_buffers(self, n: int, sieve_length: int):
-        """Two [n][sieve_length] int32 arrays for pgap_sieve, which touches the
-        head of each row: new ones are zeroed by the kernel page by page (64
-        MiB and 2.2 ms of a 3.8 ms call for 200 m's at 40000), so up to
-        LIST_BUFFER_BYTES of them are kept.  The lists are copied out."""
-        size = n * sieve_length
-        buf = self._lists
-        if buf is None or len(buf) < 2 * size:
-            buf = np.empty(2 * size, dtype=np.int32)
-            self._lists = buf if buf.nbytes <= self.LIST_BUFFER_BYTES else None
-        return buf[:size].reshape(n, sieve_length), buf[size:2 * size].reshape(n, sieve_length)
+    def _take_lists(self, size: int):
+        """An int32 array of at least `size` for pgap_sieve's lists, which fill the
+        head of each row: a new one is zeroed by the kernel page by page (64
+        MiB and 2.2 ms of a 3.8 ms call for 200 m's at 40000), so one of up to
+        LIST_BUFFER_BYTES is kept.  It belongs to the call that takes it, so calls
+        from several threads do not share one."""
+        try:
+            buf = self._lists.pop()
+        except IndexError:
+            buf = None
+        return buf if buf is not None and len(buf) >= size else np.empty(size, dtype=np.int32)
 
     def scan_config(self, depth: int, confirm: int = CONFIRM_BPSW):
         """Speculative depth cap and the confirmation (CONFIRM_*)."""
