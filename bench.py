@@ -184,7 +184,7 @@ def sieved_family_rows(engine, hipmem, P2, D2, mlo, mhi, xr, count, rng):
 MIX_UNEVEN = ((503, 210, 0.4, 1_000_000, 20000), (1511, 2190, 0.4, 1_000_000, 20000),
               (809, 1841070, 0.2, 1_000_000, 20000))
 # the uneven mix widened to the large-operand family: 3001#/2190 with m < 1e5
-# and x ~ U[-40000, 40000] (4231-4247 bits, eight lanes per number)
+# and x ~ U[-40000, 40000] (4231-4247 bits, one wavefront per number)
 MIX_WIDE = ((503, 210, 0.4, 1_000_000, 20000), (1511, 2190, 0.3, 1_000_000, 20000),
             (3001, 2190, 0.3, 100_000, 40000))
 
@@ -192,7 +192,7 @@ MIX_WIDE = ((503, 210, 0.4, 1_000_000, 20000), (1511, 2190, 0.3, 1_000_000, 2000
 def bench_mixed(engine, hipmem, pgap, count, seed, fams=MIX_UNEVEN):
     """Uneven batching: by default 40% 503#/210, 40% 1511#/2190, 20%
     809#/1841070, m ~ U[1, 1e6) coprime to d, x ~ U[-20000, 20000], no factor
-    <= 1e6, in a seeded shuffle.  Compared: one persistent launch over all
+    <= 1e6, in a seeded shuffle.  Compared: one mixed call over all
     widths, one launch per width, and every number in the widest width (one
     container)."""
     rng = np.random.default_rng(seed)
@@ -284,7 +284,8 @@ def bench_batch_family(engine, hipmem, pgap, P2, D2, m_hi, xr, count, seed, peak
                     f"candidates, {e_mean:.0f} bits",
         "tests_per_s": count / avg,
         "kernel_ms_avg": avg * 1e3,
-        "kernel": f"radix-2^{info.radix_bits} x {info.digits} digits, {info.lanes_per_number} lanes/number",
+        "kernel": "matrix cores, one wavefront/number" if info.matrix_tests == count else
+                  f"radix-2^{info.radix_bits} x {info.digits} digits, {info.lanes_per_number} lanes/number",
         "roofline_frac": 2 * L32 * L32 * e_mean * count / avg / peak_mac,
         "roofline_frac_of_nominal": 2 * L32 * L32 * e_mean * count / avg / PEAK_INT32_MAC,
         f"roofline_frac_container_{container_limbs}_limbs":
@@ -295,7 +296,7 @@ def bench_batch_family(engine, hipmem, pgap, P2, D2, m_hi, xr, count, seed, peak
 
 def bench_batch_4300(engine, hipmem, pgap, count, seed, peak_mac):
     """Large operands: N = m*3001#/2190 + x, m ~ U[1, 1e5), x ~ U[-40000,
-    40000], no factor <= 1e6 (4231-4248 bits, eight lanes per number)."""
+    40000], no factor <= 1e6 (4231-4248 bits, one wavefront per number on the matrix cores)."""
     return bench_batch_family(engine, hipmem, pgap, 3001, 2190, 100_000, 40000, count, seed, peak_mac, 136)
 
 
@@ -433,7 +434,7 @@ def main():
     ap.add_argument("--mad-peak", action="store_true", help="only measure the v_mad_u64_u32 rate")
     ap.add_argument("--no-4300", action="store_true", help="skip the 4300-bit batch")
     ap.add_argument("--batch-4300-lanes", type=int, default=0,
-                    help="lanes per number for the 4300-bit batch (0: the engine's choice, 4 lanes x 38 digits; "
+                    help="lanes per number for the 4300-bit batch (0: the engine's choice, the matrix cores; "
                          "8: the 8 x 19 variant)")
     ap.add_argument("--no-700", action="store_true", help="skip the 700-bit batch")
     ap.add_argument("--stream-m", type=int, default=16384)

@@ -11,7 +11,7 @@
 // numbers too wide for one lane and buckets of too few rows for it, run one
 // number per wavefront on the matrix cores, in one launch over all their
 // containers, widest first.  40% 705, 30% 2128 and 30% 4247 bits: 16411 numbers
-// in 28.4 ms and 131072 in 207, against 93.2 and 309 with the wide ones on 8
+// in 26.2 ms and 131072 in 191, against 93.2 and 309 with the wide ones on 8
 // lanes each and every other bucket in one-lane tiles; 2^19 narrow ones fill
 // the one-lane tiles and take 164 ms either way.
 #pragma once

@@ -1,8 +1,10 @@
 // mont_lg.h -- Montgomery arithmetic on numbers spread over a group of G
 // lanes (G = 4, 8 or 16 lanes per number), radix 2^28.
 //
-// Used where one lane cannot hold a number (above ~2240 bits the three
-// L-digit arrays of the one-lane kernel no longer fit the register file).
+// For numbers that one lane cannot hold (above ~2240 bits the three L-digit
+// arrays of the one-lane kernel no longer fit the register file) where the
+// caller fixes the lanes per number; left to choose, the engine runs those on
+// the matrix cores (mont_mf.h: 254 k tests/s at 4247 bits against 161 k).
 // Lane g of a group owns digits [g*S, (g+1)*S) of x and N; L = G*S.
 //
 // Squaring is row-wise Montgomery (CIOS): for i = 0..L-1
@@ -25,7 +27,7 @@
 // 19 digits at three.  The quad issues 17% fewer instructions per test (one
 // m broadcast per 76 products instead of per 38) and is the faster of the
 // two.  G = 16 (a whole DPP row) cuts a test's latency at a lower
-// throughput; the streaming scan uses it while few m's are in flight.
+// throughput.
 //
 // Reference counterpart: CGBN's warp-cooperative cgbn_mont_sqr with
 // TPI threads per instance (miller_rabin.h:157-211, TPI = 8 in
