@@ -166,24 +166,25 @@ __global__ void scatter_kernel(const Upload *__restrict__ up, const uint32_t *__
     }
 }
 
-// N = centre + x (side 1) or centre - x (side 0) as `w` words at o; the
-// centre has cw words (zero above).
+// N = centre + x (side 1) or centre - x (side 0) as `w` words at o, by a
+// wavefront; the centre has cw words (zero above).  A lane passes a carry on
+// when its word is all ones (all zeros for a borrow), so adding the carry into
+// the lowest lane to the mask of such lanes flips exactly the lanes that
+// receive one.
 __device__ __forceinline__ void write_n(const uint32_t *__restrict__ c, uint32_t cw, uint32_t side, uint32_t x,
-                                       uint32_t *__restrict__ o, uint32_t w) {
-    if (side) {
-        uint64_t carry = x;
-        for (uint32_t j = 0; j < w; ++j) {
-            const uint64_t v = (uint64_t)(j < cw ? c[j] : 0u) + carry;
-            o[j] = (uint32_t)v;
-            carry = v >> 32;
-        }
-    } else {
-        uint32_t borrow = x;
-        for (uint32_t j = 0; j < w; ++j) {
-            const uint32_t cj = j < cw ? c[j] : 0u;
-            o[j] = cj - borrow;
-            borrow = cj < borrow ? 1u : 0u;
-        }
+                                        uint32_t *__restrict__ o, uint32_t w) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint64_t in = 0;  // the carry into this chunk's lowest lane, or out of word 0
+    for (uint32_t base = 0; base < w; base += 64) {
+        const uint32_t j = base + lane, cj = j < cw ? c[j] : 0u;
+        const uint32_t first = side ? cj + x : cj - x;  // word 0's value
+        const bool low = j == 0;
+        uint64_t pass = __ballot(!low && cj == (side ? ~0u : 0u));
+        if (base == 0) in = (__ballot(low && (side ? first < x : cj < x)) & 1ull) << 1;
+        const uint64_t sum = pass + in, got = pass ^ sum;
+        const uint32_t one = (uint32_t)(got >> lane) & 1u;
+        if (j < w) o[j] = low ? first : (side ? cj + one : cj - one);
+        in = sum < pass ? 1u : 0u;
     }
 }
 
@@ -234,8 +235,7 @@ __global__ void count_kernel(const uint32_t *__restrict__ active, uint32_t na, c
 // One thread per (active slot, side): for a pending Fermat hit, `conf.n`
 // strong-PRP confirmation items, one per base (rows [0, cr), counter ctr[3]),
 // plus, when `lpool` is set, a strong Lucas item appended to the Lucas pool
-// (item, and its number N = centre -+ x written here: `lw` words at
-// lnum + index * lw, count *lcount); or Fermat items (rows cr + [0, ctr[0])).  Each scanning side takes its weighted share
+// (count *lcount); or Fermat items (rows cr + [0, ctr[0])).  Each scanning side takes its weighted share
 // (side_weight, total ctr[5]) of the resident lanes the confirmations (padded
 // to whole wavefronts of `cpad` items) leave, at least one, capped by `depth`
 // and by the `maxi` rows the round holds: a grid larger than the resident
@@ -243,8 +243,6 @@ __global__ void count_kernel(const uint32_t *__restrict__ active, uint32_t na, c
 __global__ void issue_kernel(const uint32_t *__restrict__ active, uint32_t na, SlotState *__restrict__ st,
                              uint32_t cr, uint32_t depth, uint32_t resident, uint32_t cpad, uint32_t maxi, Bases conf,
                              uint32_t *__restrict__ lpool, uint32_t *__restrict__ lcount, uint32_t lres,
-                             uint32_t *__restrict__ lnum, uint32_t lw, const uint32_t *__restrict__ center,
-                             uint32_t cw, const int32_t *__restrict__ lists, uint32_t cap,
                              uint32_t *__restrict__ items, uint32_t *__restrict__ item_idx,
                              uint8_t *__restrict__ item_base, uint32_t *__restrict__ ctr) {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
@@ -263,8 +261,6 @@ __global__ void issue_kernel(const uint32_t *__restrict__ active, uint32_t na, S
         if (lpool) {
             const uint32_t l = atomicAdd(lcount, 1u);
             lpool[l] = (slot << 1) | side;
-            const uint32_t x = (uint32_t)lists[((size_t)slot * 2 + side) * cap + s.cand[side]];
-            write_n(center + (size_t)slot * cw, cw, side, x, lnum + (size_t)l * lw, lw);
         }
         s.stage[side] = 0;
         s.done[side] = 0;
@@ -298,17 +294,36 @@ __device__ __forceinline__ bool row_live(uint32_t t, uint32_t cr, const uint32_t
     return t < cr ? t < ctr[3] : t - cr < ctr[0];
 }
 
-// N = centre -+ x for every item, `w` words per row.
-__global__ void materialize_kernel(const uint32_t *__restrict__ items, const uint32_t *__restrict__ item_idx,
-                                   uint32_t cr, uint32_t nrows, const uint32_t *__restrict__ ctr,
-                                   const uint32_t *__restrict__ center, uint32_t cw,
-                                   const int32_t *__restrict__ lists, uint32_t cap, uint32_t *__restrict__ nbuf,
-                                   uint32_t w) {
-    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
-    if (t >= nrows || !row_live(t, cr, ctr)) return;
-    const uint32_t slot = items[t] >> 1, side = items[t] & 1u;
-    const uint32_t x = (uint32_t)lists[((size_t)slot * 2 + side) * cap + item_idx[t]];
-    write_n(center + (size_t)slot * cw, cw, side, x, nbuf + (size_t)t * w, w);
+// N = centre -+ x for every item, `w` words per row, and behind the `nrows`
+// rows for the round's `nluc` strong Lucas items (lnum).  A wavefront per row: with a
+// thread per row, and the Lucas numbers written in the issue step, a round of
+// 1511# spent 30 + 27 us on words carried one after the other in strides of
+// a row.
+__global__ void __launch_bounds__(256) materialize_kernel(const uint32_t *__restrict__ items,
+                                                          const uint32_t *__restrict__ item_idx, uint32_t cr,
+                                                          uint32_t nrows, const uint32_t *__restrict__ ctr,
+                                                          const uint32_t *__restrict__ center, uint32_t cw,
+                                                          const int32_t *__restrict__ lists, uint32_t cap,
+                                                          uint32_t *__restrict__ nbuf, uint32_t w,
+                                                          const SlotState *__restrict__ st,
+                                                          const uint32_t *__restrict__ lpool, uint32_t nluc,
+                                                          uint32_t *__restrict__ lnum) {
+    const uint32_t t = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    uint32_t item, idx, *out;
+    if (t < nrows) {
+        if (!row_live(t, cr, ctr)) return;
+        item = items[t];
+        idx = item_idx[t];
+        out = nbuf + (size_t)t * w;
+    } else {
+        if (t - nrows >= nluc) return;
+        item = lpool[t - nrows];
+        idx = st[item >> 1].cand[item & 1u];
+        out = lnum + (size_t)(t - nrows) * w;
+    }
+    const uint32_t slot = item >> 1, side = item & 1u;
+    const uint32_t x = (uint32_t)lists[((size_t)slot * 2 + side) * cap + idx];
+    write_n(center + (size_t)slot * cw, cw, side, x, out, w);
 }
 
 // Confirmation rows count the tests their side's pending hit passed and the
@@ -1055,14 +1070,14 @@ class Scanner {
         hipLaunchKernelGGL(issue_kernel, dim3((2 * na + 255) / 256), b256, 0, stream, d_active, na, d_state, cr,
                            depth_max(), resident, cpad, maxi, conf,
                            lucas ? d_lpool + (size_t)lpool_now * LP : nullptr, lucas ? d_lctr + lpool_now : nullptr,
-                           lres, lucas ? d_lnum + (size_t)lpool_now * LP * W : nullptr, W,
-                           d_center, CW, d_lists, CAP, d_items, d_idx, d_base, d_ctr);
-        hipLaunchKernelGGL(materialize_kernel, dim3((nrows + 255) / 256), b256, 0, stream, d_items, d_idx, cr,
-                           nrows, d_ctr, d_center, CW, d_lists, CAP, d_nbuf, W);
+                           lres, d_items, d_idx, d_base, d_ctr);
+        uint32_t *lnum = lucas ? d_lnum + (size_t)lpool_now * LP * W : nullptr;
+        hipLaunchKernelGGL(materialize_kernel, dim3((nrows + nluc + 3) / 4), b256, 0, stream, d_items, d_idx, cr,
+                           nrows, d_ctr, d_center, CW, d_lists, CAP, d_nbuf, W, d_state,
+                           lucas ? d_lpool + (size_t)lpool_now * LP : nullptr, nluc, lnum);
         if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "scan issue");
         // this round's confirmations start their strong Lucas tests now,
         // beside the grid (in it, on the matrix cores)
-        const uint32_t *lnum = lucas ? d_lnum + (size_t)lpool_now * LP * W : nullptr;
         uint8_t *lverd = lucas ? d_lverd + (size_t)lpool_now * LP : nullptr;
         if (nluc && !mx && (st = lucas_launch(lpool_now, lc, nluc))) return st;
         if (mx && conf.n)
