@@ -3,7 +3,7 @@
 //
 // One wavefront per workgroup: a small batch spreads over as many compute
 // units as it has numbers.  A test costs the latency of its squarings, about
-// 1200 cycles each at 1108 bits and 1900 at 2128 (a one-lane wavefront takes
+// 1090 cycles each at 1108 bits and 1660 at 2128 (a one-lane wavefront takes
 // 12 and 43 thousand for its 64 numbers), until every SIMD has two wavefronts.
 #pragma once
 #include <algorithm>
@@ -27,7 +27,10 @@ __device__ __forceinline__ uint32_t prp_mf_test(const uint32_t *__restrict__ nw,
 
 // Wavefronts per SIMD to schedule for: the narrow widths reach four without
 // spills (1108 bits: 8.23 ms for 32768 tests against 8.59 when asked for two),
-// the wide ones would spill (2128 bits: 36.0 against 30.8 ms).
+// the wide ones would spill (2128 bits: 36.0 against 30.8 ms).  Holding only the
+// loaded fragments of N and N^-1 and spreading them at each use takes 36 to 56
+// registers off, a wavefront more per SIMD, and is slower (16384 tests: 15.4 ->
+// 17.8 ms at 2128 bits, 62 -> 69 at 4247): VALU issue bounds them, not waiting.
 constexpr int mf_waves(int KB) { return KB <= 4 ? 4 : 2; }
 
 template <int KB, int KIND>

@@ -65,6 +65,8 @@ constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may a
 // once enough sides share a round that few of its tests run past a prime.
 // Numbers too wide for one lane always run on the matrix cores.
 constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
+// Full and held: 4 and 2 take 46.5 ms for 300 m's of 1511#, 2 and 2 46.8, 3 and
+// 2 49, 4 and 1 54.
 constexpr uint32_t MATRIX_WAVES = 4;      // wavefronts per SIMD in a full matrix round
 constexpr uint32_t MATRIX_WAVES_HELD = 2;  // ... while few sides scan
 constexpr uint32_t LUCAS_LANES = 128;     // of a strong Lucas test on the matrix cores
