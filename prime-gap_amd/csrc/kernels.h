@@ -4,6 +4,7 @@
 // instantiation unit (prp_r28_*.hip, ...) registers the variants it compiles;
 // the engine picks the smallest variant whose digits cover a batch.
 #pragma once
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
@@ -87,6 +88,14 @@ typedef hipError_t (*matrix_scan_fn)(const uint32_t *d_n, uint32_t limbs, uint32
                                      uint32_t max_items, const uint32_t *d_ctr, const uint8_t *d_base,
                                      uint8_t *d_out, const uint32_t *d_lnum, uint32_t nluc, uint8_t *d_lverd,
                                      hipStream_t stream);
+
+// Workgroups of a matrix-core launch whose count the host knows: one per number,
+// so that the dispatcher evens out their times, up to this.  A dispatch takes
+// fewer than 2^32 threads, 2^25 workgroups of 128, and a chunk has up to 2^30
+// numbers: past the cap a workgroup of a batch tests every 2^22nd, and a mixed
+// call launches again.
+constexpr uint32_t kMatrixMaxBlocks = 1u << 22;
+inline uint32_t matrix_blocks(uint32_t rows) { return std::min(rows, kMatrixMaxBlocks); }
 
 struct MatrixVariant {
     int blocks;    // 16-word blocks of the number's container (mont_mf.h's KB)

@@ -207,7 +207,7 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
     e->last.digits = 0;
     e->last.radix_bits = 28;
     e->last.lanes_per_number = 0;  // per bucket
-    e->last.launches = (nmx ? 1u : 0u) + (ntiles ? 1u : 0u);
+    e->last.launches = (uint32_t)((nmx + kMatrixMaxBlocks - 1ull) / kMatrixMaxBlocks) + (ntiles ? 1u : 0u);
     e->last.tests = count;
     e->last.matrix_tests = nmx;
     e->timing_pending = true;

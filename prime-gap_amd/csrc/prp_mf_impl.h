@@ -53,7 +53,7 @@ hipError_t launch_mf(const uint32_t *d_n, uint32_t limbs, uint32_t first, uint32
                      const uint32_t *d_count, const uint32_t *d_idx, uint32_t base, uint8_t *d_out,
                      hipStream_t stream) {
     if (first >= count) return hipSuccess;
-    const uint32_t blocks = d_count ? std::min(count, kMatrixBlocks) : count - first;
+    const uint32_t blocks = d_count ? std::min(count, kMatrixBlocks) : matrix_blocks(count - first);
     hipLaunchKernelGGL((prp_mf_kernel<KB, KIND>), dim3(blocks), dim3(64), 0, stream, d_n, limbs, first, count, d_first,
                        d_count, d_idx, base, d_out);
     return hipGetLastError();
@@ -124,7 +124,7 @@ hipError_t launch_lucas_mf(const uint32_t *d_n, uint32_t limbs, uint32_t first, 
                            const uint32_t *d_first, const uint32_t *d_count, const uint32_t *d_idx, uint32_t,
                            uint8_t *d_out, hipStream_t stream) {
     if (first >= count) return hipSuccess;
-    const uint32_t blocks = d_count ? std::min(count, kMatrixBlocks) : count - first;
+    const uint32_t blocks = d_count ? std::min(count, kMatrixBlocks) : matrix_blocks(count - first);
     hipLaunchKernelGGL((lucas_mf_kernel<KB>), dim3(blocks), dim3(128), 0, stream, d_n, limbs, first, count, d_first,
                        d_count, d_idx, d_out);
     return hipGetLastError();
