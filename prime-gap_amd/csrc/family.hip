@@ -70,16 +70,21 @@ __device__ __forceinline__ bool fits_fixed(uint64_t m, int64_t x) {
     return m < (1ull << 32) && x >= -(1ll << 31) && x < (1ll << 31);
 }
 
-// A candidate of the prime-parallel stages: (m, x + 2^31) and its row.
+// The candidates of the prime-parallel stages.  The fixed-point ones fill the
+// arrays from the front: (m, x + 2^31) and the row.  Those outside its range (m
+// >= 2^32 or |x| >= 2^31) fill `row` from the back, `end` being its end: a
+// candidate is on one of the two lists.
 struct Listed {
     uint2 *pair;
-    uint32_t *row, *n;
+    uint32_t *row, *end;
+    uint32_t *n, *n_wide;
 };
 
-// Appends the flagged threads' candidates, one global atomic per workgroup of
-// 1024 (a counter takes one about every 10 ns: per wavefront, 2^20 candidates
-// spent 0.16 ms of the stage's 0.20 on it).
-__device__ __forceinline__ void append(bool flag, uint2 pair, uint32_t row, const Listed &out) {
+// Calls put(place) in the flagged threads, places counted from *n: one global
+// atomic per workgroup of 1024 (a counter takes one about every 10 ns: per
+// wavefront, 2^20 candidates spent 0.16 ms of the stage's 0.20 on it).
+template <class Put>
+__device__ __forceinline__ void append(bool flag, uint32_t *n, const Put &put) {
     __shared__ uint32_t total, base;
     if (threadIdx.x == 0) total = 0;
     __syncthreads();
@@ -89,22 +94,25 @@ __device__ __forceinline__ void append(bool flag, uint2 pair, uint32_t row, cons
     if (lane == 0) at = atomicAdd(&total, (uint32_t)__popcll(mask));
     at = (uint32_t)__shfl((int)at, 0, 64) + (uint32_t)__popcll(mask & ((1ull << lane) - 1));
     __syncthreads();
-    if (threadIdx.x == 0) base = total ? atomicAdd(out.n, total) : 0u;
+    if (threadIdx.x == 0) base = total ? atomicAdd(n, total) : 0u;
     __syncthreads();
-    if (flag) {
-        out.pair[base + at] = pair;
-        out.row[base + at] = row;
-    }
+    if (flag) put(base + at);
+}
+// Both lists; most calls have no wide candidate.
+__device__ __forceinline__ void append(bool fixed, uint2 pair, bool wide, uint32_t row, const Listed &out) {
+    append(fixed, out.n, [&](uint32_t at) {
+        out.pair[at] = pair;
+        out.row[at] = row;
+    });
+    if (__syncthreads_or(wide)) append(wide, out.n_wide, [&](uint32_t at) { out.end[-1 - (int64_t)at] = row; });
 }
 
 // First stage: a thread per candidate over the primes below 2^10 (table
 // [0, k1), which the scalar cache holds).  Survivors are kept and listed for
-// the prime-parallel stages.  A candidate too large for the fixed-point test
-// meets every prime here, exactly.
+// the prime-parallel stages.
 __global__ void __launch_bounds__(1024) filter_first_kernel(const uint64_t *__restrict__ m, const int64_t *__restrict__ x,
                                                             uint32_t count, const FilterPrime *__restrict__ table,
-                                                            uint32_t k1, uint32_t np, uint8_t *__restrict__ keep,
-                                                            Listed out) {
+                                                            uint32_t k1, uint8_t *__restrict__ keep, Listed out) {
     const uint32_t i = blockIdx.x * 1024u + threadIdx.x;
     const uint64_t mi = i < count ? m[i] : 0u;
     const int64_t xi = i < count ? x[i] : 0;
@@ -121,21 +129,29 @@ __global__ void __launch_bounds__(1024) filter_first_kernel(const uint64_t *__re
             alive = min(min(high(k), high(k + 1)), min(high(k + 2), high(k + 3))) > kMarginTop;
         for (; alive && k < k1; ++k) alive = high(k) > kMarginTop;
     } else {
-        for (uint32_t k = 0; alive && k < np; ++k) alive = !divides(table[k], mi, xi);
+        for (uint32_t k = 0; alive && k < k1; ++k) alive = !divides(table[k], mi, xi);
     }
     if (i < count) keep[i] = alive ? 1 : 0;
-    append(alive && fixed, make_uint2(m32, xs), i, out);
+    append(alive && fixed, make_uint2(m32, xs), alive && !fixed, i, out);
 }
 
 // The listed candidates still kept.
 __global__ void __launch_bounds__(1024) filter_compact_kernel(const uint8_t *__restrict__ keep, Listed in, Listed out) {
-    const uint32_t n = *in.n;
-    for (uint32_t c0 = blockIdx.x * 1024u; c0 < n; c0 += gridDim.x * 1024u) {
+    const uint32_t n = *in.n, nw = *in.n_wide;
+    for (uint32_t c0 = blockIdx.x * 1024u; c0 < max(n, nw); c0 += gridDim.x * 1024u) {
         const uint32_t c = c0 + threadIdx.x;
-        const uint2 pair = c < n ? in.pair[c] : make_uint2(0, 0);
-        const uint32_t row = c < n ? in.row[c] : 0u;
-        append(c < n && keep[row], pair, row, out);
-        __syncthreads();
+        if (c0 < n) {
+            const uint2 pair = c < n ? in.pair[c] : make_uint2(0, 0);
+            const uint32_t row = c < n ? in.row[c] : 0u;
+            append(c < n && keep[row], out.n, [&](uint32_t at) {
+                out.pair[at] = pair;
+                out.row[at] = row;
+            });
+        }
+        if (c0 < nw) {
+            const uint32_t row = c < nw ? in.end[-1 - (int64_t)c] : 0u;
+            append(c < nw && keep[row], out.n_wide, [&](uint32_t at) { out.end[-1 - (int64_t)at] = row; });
+        }
     }
 }
 
@@ -146,16 +162,20 @@ __global__ void __launch_bounds__(1024) filter_compact_kernel(const uint8_t *__r
 // (8.3 10^12 a second, the multiply-add rate); a thread per candidate with
 // Barrett reductions kept 1.3 wavefronts per SIMD busy for 28.0 ms, and the
 // primes below 2^15 for 1.27 ms (0.53 in fixed point, waiting for the table).
-__global__ void __launch_bounds__(256) filter_primes_kernel(const uint2 *__restrict__ pair, const uint32_t *__restrict__ idx,
-                                                          const uint32_t *__restrict__ n_in,
-                                                          const FilterPrime *__restrict__ table, uint32_t k0,
+// Candidates outside the fixed-point range take three Barrett reductions a
+// prime in the same split: 2^20 pairs with m above 2^33 in a call of 7.6 ms, against
+// 30.2 with a thread per compacted candidate and 146 with a thread per
+// candidate over the whole table.
+__global__ void __launch_bounds__(256) filter_primes_kernel(const uint64_t *__restrict__ m, const int64_t *__restrict__ x,
+                                                          Listed in, const FilterPrime *__restrict__ table, uint32_t k0,
                                                           uint32_t k1, uint8_t *__restrict__ keep) {
-    const uint32_t k = k0 + blockIdx.x * 256u + threadIdx.x, n = *n_in;
+    const uint2 *__restrict__ pair = in.pair;
+    const uint32_t k = k0 + blockIdx.x * 256u + threadIdx.x, n = *in.n, nw = *in.n_wide;
     if (k >= k1) return;
     const FilterPrime f = table[k];
     const auto clear = [&](uint32_t c, uint32_t high) {
         if (high <= kMarginTop && (f.p < kFixedExact || divides(f, pair[c].x, (int64_t)pair[c].y - (1ll << 31))))
-            keep[idx[c]] = 0;
+            keep[in.row[c]] = 0;
     };
     for (uint32_t c = 8 * blockIdx.y; c < n; c += 8 * gridDim.y) {
         if (c + 8 > n) {
@@ -171,6 +191,10 @@ __global__ void __launch_bounds__(256) filter_primes_kernel(const uint2 *__restr
         if (least > kMarginTop) continue;
 #pragma unroll
         for (uint32_t j = 0; j < 8; ++j) clear(c + j, high[j]);
+    }
+    for (uint32_t c = blockIdx.y; c < nw; c += gridDim.y) {
+        const uint32_t row = in.end[-1 - (int64_t)c];
+        if (divides(f, m[row], x[row])) keep[row] = 0;
     }
 }
 
@@ -379,25 +403,27 @@ pgap_status pgap_filter_candidates(pgap_engine *e, int family, const uint64_t *m
         (he = hipMemsetAsync(e->d_small.p, 0, 16, e->stream)) != hipSuccess)
         return e->hip_fail(he, "filter upload");
     // primes < 2^10, < 2^15, the rest; survivors are compacted between them
-    // (counters in d_small[0], d_small[1])
+    // (counters in d_small: [0], [1], and [2], [3] for the wide candidates)
     const uint32_t np = (uint32_t)f->nprimes;
     const uint32_t e0 = std::min(f->stage_end[0], np), e1 = std::min(f->stage_end[1], np);
     const auto listed = [&](DevBuf &b, int k) {
-        return Listed{(uint2 *)b.p, (uint32_t *)((uint2 *)b.p + count), (uint32_t *)e->d_small.p + k};
+        uint32_t *row = (uint32_t *)((uint2 *)b.p + count), *n = (uint32_t *)e->d_small.p + k;
+        return Listed{(uint2 *)b.p, row, row + count, n, n + 2};
     };
     const Listed la = listed(e->d_idx0, 0), lb = listed(e->d_idx1, 1);
+    const uint64_t *d_m = (const uint64_t *)e->d_m.p;
+    const int64_t *d_x = (const int64_t *)e->d_x.p;
     uint8_t *d_keep = (uint8_t *)e->d_keep.p;
-    hipLaunchKernelGGL(filter_first_kernel, dim3((uint32_t)((count + 1023) / 1024)), dim3(1024), 0, e->stream,
-                       (const uint64_t *)e->d_m.p, (const int64_t *)e->d_x.p, (uint32_t)count, f->d_filter, e0, np,
-                       d_keep, la);
+    hipLaunchKernelGGL(filter_first_kernel, dim3((uint32_t)((count + 1023) / 1024)), dim3(1024), 0, e->stream, d_m, d_x,
+                       (uint32_t)count, f->d_filter, e0, d_keep, la);
     if (e0 < e1)
-        hipLaunchKernelGGL(filter_primes_kernel, dim3((e1 - e0 + 255) / 256, 512), dim3(256), 0, e->stream, la.pair,
-                           la.row, la.n, f->d_filter, e0, e1, d_keep);
+        hipLaunchKernelGGL(filter_primes_kernel, dim3((e1 - e0 + 255) / 256, 512), dim3(256), 0, e->stream, d_m, d_x,
+                           la, f->d_filter, e0, e1, d_keep);
     if (e1 < np) {
         hipLaunchKernelGGL(filter_compact_kernel, dim3((uint32_t)std::min<size_t>((count + 1023) / 1024, 512)),
                            dim3(1024), 0, e->stream, d_keep, la, lb);
-        hipLaunchKernelGGL(filter_primes_kernel, dim3((np - e1 + 255) / 256, 64), dim3(256), 0, e->stream, lb.pair,
-                           lb.row, lb.n, f->d_filter, e1, np, d_keep);
+        hipLaunchKernelGGL(filter_primes_kernel, dim3((np - e1 + 255) / 256, 64), dim3(256), 0, e->stream, d_m, d_x, lb,
+                           f->d_filter, e1, np, d_keep);
     }
     if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "filter kernels");
     if ((he = hipMemcpyAsync(keep, e->d_keep.p, count, hipMemcpyDeviceToHost, e->stream)) != hipSuccess ||
