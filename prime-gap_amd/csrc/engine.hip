@@ -552,6 +552,7 @@ void pgap_destroy(pgap_engine *e) {
         (void)hipStreamSynchronize(e->stream);
         e->scan_shutdown();
         e->sieve_shutdown();
+        if (e->sieve_stage) (void)hipHostFree(e->sieve_stage);
         e->families_shutdown();
         if (e->graph.exec) (void)hipGraphExecDestroy(e->graph.exec);
         e->graph.exec = nullptr;
