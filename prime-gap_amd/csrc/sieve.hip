@@ -285,15 +285,17 @@ __global__ void __launch_bounds__(256) sieve_count_kernel(const uint32_t *__rest
     if (threadIdx.x == 0) counts[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
 }
 
-// Their distances, each list at offsets[workgroup] of out: a workgroup takes
-// 256 words of its side at a time, scans their counts and scatters.
+// Their distances, each list at offsets[workgroup] of out, or at workgroup * SL
+// with its length in counts where there are no offsets: a workgroup takes 256
+// words of its side at a time, scans their counts and scatters.
 __global__ void __launch_bounds__(256) sieve_list_kernel(const uint32_t *__restrict__ bitmap, uint32_t words,
                                                          uint32_t SL, const uint32_t *__restrict__ offsets,
-                                                         int32_t *__restrict__ out) {
+                                                         uint32_t *__restrict__ counts, int32_t *__restrict__ out) {
     __shared__ uint32_t part[4];
     const uint32_t *bm = bitmap + (size_t)(blockIdx.x >> 1) * words;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t done = offsets[blockIdx.x];
+    const uint32_t start = offsets ? offsets[blockIdx.x] : blockIdx.x * SL;
+    uint32_t done = start;
     for (uint32_t t0 = 0; 32 * t0 < SL; t0 += 256) {
         const uint32_t t = t0 + threadIdx.x;
         uint32_t w = 32 * t < SL ? side_word(bm, words, SL, blockIdx.x & 1u, t) : 0u;
@@ -314,6 +316,7 @@ __global__ void __launch_bounds__(256) sieve_list_kernel(const uint32_t *__restr
             w &= w - 1;
         }
     }
+    if (!offsets && threadIdx.x == 0) counts[blockIdx.x] = done - start;
 }
 
 }  // namespace pgap
@@ -331,6 +334,12 @@ static void free_small(Family &f) {
 // does not depend on the limit: freed with the prime tables at each change of it,
 // two calls of 4 m's to 1e8 and 1e7 in turn took 12.1 ms.
 constexpr size_t STAGE_WORDS = (size_t)8 << 20;
+// Up to so many words of full lists, a batch's lists come back at their full
+// length with their counts: one wait instead of a count kernel, a wait for the
+// lengths and an upload of the places.  Whole calls, us, that way against the
+// other: 200 words (one m, SL = 100, to 1000) 38 / 65, 32000 78 / 95, 128000 95 /
+// 102, 160000 188 / 204, 480000 215 / 210, 1024000 245 / 200.
+constexpr size_t DIRECT_WORDS = (size_t)1 << 18;
 
 void pgap_engine::sieve_shutdown() {
     if (sieve_primes) (void)hipFree(sieve_primes);
@@ -485,17 +494,18 @@ extern "C" pgap_status pgap_sieve(pgap_engine *e, int family, const uint64_t *m,
     hipLaunchKernelGGL(sieve_base_kernel, dim3((words + SMALL_SEG - 1) / SMALL_SEG), dim3(256), 0, e->stream, SL, sp,
                        skm, f->nsmall, words, base);
     if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "sieve base kernel");
-    std::vector<uint32_t> len(2 * batch), at(2 * batch), m32(batch);
+    std::vector<uint32_t> len(2 * batch), at(2 * batch), up(3 * batch);  // up: the m's, then their low words
     uint32_t *d_m32 = (uint32_t *)((uint64_t *)e->d_m.p + batch);
     for (size_t off = 0; off < count; off += batch) {
         const uint32_t nb = (uint32_t)std::min(batch, count - off);
         uint64_t m_max = 0;
         for (uint32_t j = 0; j < nb; ++j) {
             m_max = std::max(m_max, m[off + j]);
-            m32[j] = (uint32_t)m[off + j];
+            up[2 * batch + j] = (uint32_t)m[off + j];
         }
-        if ((he = hipMemcpyAsync(e->d_m.p, m + off, nb * 8, hipMemcpyHostToDevice, e->stream)) != hipSuccess ||
-            (he = hipMemcpyAsync(d_m32, m32.data(), nb * 4, hipMemcpyHostToDevice, e->stream)) != hipSuccess)
+        memcpy(up.data(), m + off, nb * 8);
+        if ((he = hipMemcpyAsync(e->d_m.p, up.data(), (2 * batch + nb) * 4, hipMemcpyHostToDevice, e->stream)) !=
+            hipSuccess)
             return e->hip_fail(he, "sieve m upload");
         hipLaunchKernelGGL(sieve_small_kernel, dim3(nb), dim3(1024), words * 4, e->stream,
                            (const uint64_t *)e->d_m.p, SL, sp, skm, f->d_small, f->nsmall, f->nsmall_wave, words,
@@ -507,6 +517,26 @@ extern "C" pgap_status pgap_sieve(pgap_engine *e, int family, const uint64_t *m,
             const auto large = fixed ? &sieve_large_kernel<true> : &sieve_large_kernel<false>;
             hipLaunchKernelGGL(large, dim3(grid), dim3(256), 0, e->stream, (const uint64_t *)e->d_m.p, d_m32, nb, m_max, SL,
                                e->sieve_primes, f->d_skmod, e->sieve_mu, e->sieve_nprimes, words, (uint32_t *)bm.p);
+        }
+        if (const size_t full = (size_t)2 * nb * SL; full <= DIRECT_WORDS) {
+            if ((st = e->ensure(e->d_x, (full + 2 * nb) * 4, "lists"))) return st;
+            uint32_t *counts = (uint32_t *)e->d_x.p + full;
+            hipLaunchKernelGGL(sieve_list_kernel, dim3(2 * nb), dim3(256), 0, e->stream, (const uint32_t *)bm.p, words,
+                               SL, nullptr, counts, (int32_t *)e->d_x.p);
+            if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "sieve kernels");
+            if ((he = hipMemcpyAsync(e->sieve_stage, e->d_x.p, (full + 2 * nb) * 4, hipMemcpyDeviceToHost,
+                                     e->stream)) != hipSuccess ||
+                (he = hipStreamSynchronize(e->stream)) != hipSuccess)
+                return e->hip_fail(he, "sieve readback");
+            for (uint32_t j = 0; j < nb; ++j) {
+                const size_t i = off + j;
+                const uint32_t *list = e->sieve_stage + (size_t)2 * j * SL;
+                n_prev[i] = e->sieve_stage[full + 2 * j];
+                n_next[i] = e->sieve_stage[full + 2 * j + 1];
+                memcpy(prev + i * SL, list, (size_t)n_prev[i] * 4);
+                memcpy(next + i * SL, list + SL, (size_t)n_next[i] * 4);
+            }
+            continue;
         }
         hipLaunchKernelGGL(sieve_count_kernel, dim3(2 * nb), dim3(256), 0, e->stream, (const uint32_t *)bm.p, words,
                            SL, (uint32_t *)e->d_idx0.p);
@@ -531,7 +561,7 @@ extern "C" pgap_status pgap_sieve(pgap_engine *e, int family, const uint64_t *m,
                 return e->hip_fail(he, "sieve offsets");
             hipLaunchKernelGGL(sieve_list_kernel, dim3(2 * (j1 - j0)), dim3(256), 0, e->stream,
                                (const uint32_t *)bm.p + (size_t)j0 * words, words, SL,
-                               (const uint32_t *)e->d_idx1.p, (int32_t *)e->d_x.p);
+                               (const uint32_t *)e->d_idx1.p, nullptr, (int32_t *)e->d_x.p);
             if ((he = hipGetLastError()) != hipSuccess) return e->hip_fail(he, "sieve list kernel");
             if ((total && (he = hipMemcpyAsync(e->sieve_stage, e->d_x.p, total * 4, hipMemcpyDeviceToHost,
                                                e->stream)) != hipSuccess) ||
