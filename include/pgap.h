@@ -242,11 +242,15 @@ pgap_status pgap_scan_stats(const pgap_engine *e, uint64_t *tests_issued, uint64
 /* Autotuner.  For each width in bits[0..n), times every kernel family that
  * covers it (one lane per number; a group of 4, 8 or 16 lanes per number;
  * radix 2^28) at its smallest covering size and under a few occupancy caps,
- * for each test (Fermat, strong PRP, strong Lucas), and keeps the fastest.
+ * for each test (Fermat, strong PRP, strong Lucas), keeps the fastest, and times
+ * the matrix cores beside it.
  * The table replaces the engine's
  * current one (later batches and scans use it) and, when path is non-NULL,
  * is written there for pgap_options.tuning_path.  Text format, one line per
- * (test, width): "<test> <max_bits> <radix> <digits> <lanes> <cap> <tests/s>".
+ * (test, width): "<test> <max_bits> <radix> <digits> <lanes> <cap> <tests/s>
+ * <matrix tests/s>".  A lane group runs every row unless its entry has the
+ * matrix cores faster (a table without the last field has not); one lane per
+ * number runs whole rounds of the device, and the matrix cores the remainder.
  * Replaces the reference's compile-time choice of BITS / WINDOW_BITS /
  * THREADS_PER_INSTANCE (gap_test_gpu.cu:48-81). */
 pgap_status pgap_autotune(pgap_engine *e, const uint32_t *bits, size_t n, const char *path);

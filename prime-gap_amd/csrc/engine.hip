@@ -155,7 +155,16 @@ Choice pgap_engine::select(int kind, uint32_t bits) const {
     Choice c;
     std::lock_guard<std::mutex> g(tune_mu);
     const TuneEntry *t = (opt.radix || opt.lanes_per_number) ? nullptr : tuned(kind, bits);
-    if (t) c.v = find_variant(kind, (int)bits, t->radix, t->lanes);
+    if (t && (c.v = find_variant(kind, (int)bits, t->radix, t->lanes))) {
+        c.table = t->matrix_rate > t->rate ? Choice::TABLE_MATRIX : Choice::TABLE_VECTOR;
+        // an entry's group and its matrix rate are of the entry's width: numbers
+        // that fit one lane keep the rule of plan()
+        const Variant *one = find_variant(kind, (int)bits, 0, 1);
+        if (c.table == Choice::TABLE_MATRIX && c.v->lanes != 1 && one) {
+            c.v = one;
+            c.table = Choice::NO_TABLE;
+        }
+    }
     if (!c.v) c.v = find_variant(kind, (int)bits, opt.radix, opt.lanes_per_number);
     if (!c.v && (opt.radix || opt.lanes_per_number)) c.v = find_variant(kind, (int)bits, 0, 0);
     if (!c.v) return c;
@@ -190,7 +199,9 @@ pgap_status pgap_engine::pick(int kind, uint32_t bits, Choice *out) {
 // their count: 20000 of 4247 bits in 78 ms against 199 on 4 lanes each.  Below
 // kMatrixMinBits the set-up of a number on a whole wavefront costs more than
 // its squarings save.  A caller that forces a radix, lanes or an occupancy
-// keeps the lane kernels.
+// keeps the lane kernels, and so does a tuning table whose entry is a lane group
+// unless it has the matrix cores faster; a one-lane entry's remainders follow
+// the rule above (the table holds rates of full launches, not latencies).
 constexpr uint32_t kMatrixCycles[6] = {0, 400, 480, 590, 710, 1110};  // by container
 
 uint32_t pgap_engine::matrix_limit(int digits, int blocks) const {
@@ -202,9 +213,9 @@ pgap_status pgap_engine::plan(int kind, uint32_t bits, const Bases &bases, Plan 
     *out = Plan{};
     pgap_status st;
     if ((st = pick(kind, select_bits(kind, bits, bases), &out->lane))) return st;
-    if (forced() || (kind != KIND_LUCAS && bits < kMatrixMinBits)) return PGAP_OK;
+    if (forced() || out->lane.tuned_group() || (kind != KIND_LUCAS && bits < kMatrixMinBits)) return PGAP_OK;
     out->mx = find_matrix(kind, (int)bits);
-    if (!out->mx || out->lane.v->lanes != 1) return PGAP_OK;
+    if (!out->mx || out->lane.v->lanes != 1 || out->lane.table == Choice::TABLE_MATRIX) return PGAP_OK;
     out->round = 256u * (uint32_t)num_cus;
     out->limit = matrix_limit(out->lane.v->digits, out->mx->blocks);
     return PGAP_OK;

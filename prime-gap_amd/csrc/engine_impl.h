@@ -21,12 +21,13 @@ struct DevBuf {
 class Scanner;
 
 // One autotuner decision: numbers of up to `bits` bits of test `kind` run on
-// the variant (radix, digits, lanes) with an occupancy cap.
+// the variant (radix, digits, lanes) with an occupancy cap, or on the matrix
+// cores if these were timed faster (matrix_rate 0: not timed).
 struct TuneEntry {
     int kind = 0;
     uint32_t bits = 0;
     int radix = 0, digits = 0, lanes = 0, blocks_cap = 0;
-    double rate = 0;
+    double rate = 0, matrix_rate = 0;
 };
 
 // Rows per batch launch: grid dimensions are 32-bit.
@@ -36,6 +37,9 @@ constexpr size_t kBatchChunk = (size_t)1 << 30;
 struct Choice {
     const Variant *v = nullptr;
     int cap = 0;
+    enum { NO_TABLE, TABLE_VECTOR, TABLE_MATRIX } table = NO_TABLE;  // what a tuning table has as the fastest
+    // A lane group that a table prefers to the matrix cores.
+    bool tuned_group() const { return table == TABLE_VECTOR && v->lanes != 1; }
 };
 
 // Narrowest batch for the matrix cores (see plan()).

@@ -63,7 +63,8 @@ constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may a
 // window; above the threshold the one-lane rounds take over, which test more
 // numbers a second (at 2128 bits 1.56 against 1.0 M/s, but in rounds of 42 ms)
 // once enough sides share a round that few of its tests run past a prime.
-// Numbers too wide for one lane always run on the matrix cores.
+// Numbers too wide for one lane run on the matrix cores whatever their count,
+// unless a tuning table has a lane group faster.
 constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
 // Full and held: 4 and 2 take 46.5 ms for 300 m's of 1511#, 2 and 2 46.8, 3 and
 // 2 49, 4 and 1 54.
@@ -1001,7 +1002,7 @@ class Scanner {
         // sides that will scan this round (m's waiting for confirmations do not)
         const uint32_t sides = (uint32_t)std::min<uint64_t>(2ull * na, (uint64_t)last_scanning + 2ull * admitted_last);
         const MatrixVariant *mx = nullptr;  // of the round's strong-PRP and Fermat rows
-        if (!e->forced() && (cf.v->lanes > 1 || sides <= LATENCY_SIDES))
+        if (!e->forced() && ((cf.v->lanes > 1 && !cf.tuned_group()) || sides <= LATENCY_SIDES))
             mx = find_matrix(conf.n ? KIND_SPRP : KIND_FERMAT2, (int)bits);
         const Variant *vf = cf.v, *vc = cc.v;
         if (vc && !vc->scan) {
@@ -1065,7 +1066,9 @@ class Scanner {
             if (nluc && mx) {
                 lres = LUCAS_LANES;
             } else if (nluc) {
-                if ((st = e->plan(KIND_LUCAS, bits, none, &lc))) return st;
+                // one kernel for every round's Lucas tests, whatever a table has for batches
+                if (!e->forced()) lc.mx = find_matrix(KIND_LUCAS, (int)bits);
+                if (!lc.mx && (st = e->plan(KIND_LUCAS, bits, none, &lc))) return st;
                 lres = resident < resident_full ? (lc.mx ? LUCAS_LANES : (uint32_t)lc.lane.v->lanes) : 0u;
             }
         }

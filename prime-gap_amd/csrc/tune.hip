@@ -1,7 +1,7 @@
 // tune.hip -- the autotuner: for each number width, time every kernel family
 // (one lane per number, a group of 4, 8 or 16 lanes per number; radix 2^28) at its
 // smallest covering digit count and under a few occupancy caps, and keep the
-// fastest.  The table is plain text and is loaded by pgap_create through
+// fastest, with the rate of the matrix cores beside it.  The table is plain text and is loaded by pgap_create through
 // pgap_options.tuning_path.
 //
 // Reference counterpart: none in code -- the reference fixes BITS,
@@ -11,9 +11,10 @@
 // the small strong-PRP bases never use a table.
 //
 // Table format, one entry per line:
-//   <kind> <max_bits> <radix> <digits> <lanes> <blocks_cap> <tests_per_s>
+//   <kind> <max_bits> <radix> <digits> <lanes> <blocks_cap> <tests_per_s> <matrix_tests_per_s>
 // kind 0 = Fermat base 2, 1 = strong PRP, 2 = strong Lucas; blocks_cap 0 =
-// natural occupancy.
+// natural occupancy; the last field is 0 where the matrix cores do not run, and
+// missing from tables that were written without it.
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -31,8 +32,8 @@ bool pgap_engine::load_tuning(const char *path) {
     while (fgets(line, sizeof line, f)) {
         if (line[0] == '#') continue;
         TuneEntry t{};
-        if (sscanf(line, "%d %u %d %d %d %d %lf", &t.kind, &t.bits, &t.radix, &t.digits, &t.lanes, &t.blocks_cap,
-                   &t.rate) == 7)
+        if (sscanf(line, "%d %u %d %d %d %d %lf %lf", &t.kind, &t.bits, &t.radix, &t.digits, &t.lanes, &t.blocks_cap,
+                   &t.rate, &t.matrix_rate) >= 7)
             tune.push_back(t);
     }
     fclose(f);
@@ -95,33 +96,46 @@ extern "C" pgap_status pgap_autotune(pgap_engine *e, const uint32_t *bits, size_
                 bs.n = 1;
                 bs.b[0] = 3;
             }
-            for (const Variant *v : cand) {
-                const int natural = v->blocks_per_cu ? v->blocks_per_cu() : 1;
-                const size_t count = (size_t)std::max(1, natural) * e->num_cus * 256 / (size_t)v->lanes * 2;
+            // the second of two launches over `count` random numbers, in tests/s
+            const auto upload = [&](size_t count) -> pgap_status {
                 fill_random(host, count, limbs, b, 0x9e3779b97f4a7c15ull ^ b);
                 pgap_status st;
                 if ((st = e->ensure(e->d_n, host.size() * 4, "tuning numbers")) ||
                     (st = e->ensure(e->d_out, count, "tuning verdicts")))
                     return st;
                 hipError_t he = hipMemcpy(e->d_n.p, host.data(), host.size() * 4, hipMemcpyHostToDevice);
-                if (he != hipSuccess) return e->hip_fail(he, "tuning upload");
+                return he == hipSuccess ? PGAP_OK : e->hip_fail(he, "tuning upload");
+            };
+            const auto time = [&](size_t count, const auto &launch, double *rate) -> pgap_status {
+                float best_ms = 1e30f;
+                for (int rep = 0; rep < 2; ++rep) {
+                    hipError_t he;
+                    if ((he = hipEventRecord(e->ev0, e->stream)) != hipSuccess || (he = launch()) != hipSuccess ||
+                        (he = hipEventRecord(e->ev1, e->stream)) != hipSuccess ||
+                        (he = hipEventSynchronize(e->ev1)) != hipSuccess)
+                        return e->hip_fail(he, "tuning launch");
+                    float ms = 0;
+                    (void)hipEventElapsedTime(&ms, e->ev0, e->ev1);
+                    if (rep) best_ms = std::min(best_ms, ms);
+                }
+                *rate = count / (best_ms * 1e-3);
+                return PGAP_OK;
+            };
+            pgap_status st;
+            for (const Variant *v : cand) {
+                const int natural = v->blocks_per_cu ? v->blocks_per_cu() : 1;
+                const size_t count = (size_t)std::max(1, natural) * e->num_cus * 256 / (size_t)v->lanes * 2;
+                if ((st = upload(count))) return st;
                 std::vector<int> caps = {0};
                 if (natural > 1) caps.push_back(1);
                 if (natural > 2) caps.push_back(natural - 1);
                 for (int cap : caps) {
-                    float best_ms = 1e30f;
-                    for (int rep = 0; rep < 2; ++rep) {
-                        if ((he = hipEventRecord(e->ev0, e->stream)) != hipSuccess ||
-                            (he = v->launch((const uint32_t *)e->d_n.p, limbs, (uint32_t)count, nullptr, nullptr, bs,
-                                            (uint8_t *)e->d_out.p, cap, e->stream)) != hipSuccess ||
-                            (he = hipEventRecord(e->ev1, e->stream)) != hipSuccess ||
-                            (he = hipEventSynchronize(e->ev1)) != hipSuccess)
-                            return e->hip_fail(he, "tuning launch");
-                        float ms = 0;
-                        (void)hipEventElapsedTime(&ms, e->ev0, e->ev1);
-                        if (rep) best_ms = std::min(best_ms, ms);
-                    }
-                    const double rate = count / (best_ms * 1e-3);
+                    double rate;
+                    const auto launch = [&] {
+                        return v->launch((const uint32_t *)e->d_n.p, limbs, (uint32_t)count, nullptr, nullptr, bs,
+                                         (uint8_t *)e->d_out.p, cap, e->stream);
+                    };
+                    if ((st = time(count, launch, &rate))) return st;
                     if (rate > best.rate) {
                         best.kind = kind;
                         best.bits = b;
@@ -133,6 +147,17 @@ extern "C" pgap_status pgap_autotune(pgap_engine *e, const uint32_t *bits, size_
                     }
                 }
             }
+            // the matrix cores, at widths where plan() uses them
+            const MatrixVariant *mx = find_matrix(kind, (int)b);
+            if (mx && (kind == KIND_LUCAS || b >= kMatrixMinBits)) {
+                const size_t count = 64 * (size_t)e->num_cus;  // 16 per SIMD, several rounds of the resident ones
+                if ((st = upload(count))) return st;
+                const auto launch = [&] {
+                    return mx->launch((const uint32_t *)e->d_n.p, limbs, 0, (uint32_t)count, nullptr, nullptr, nullptr,
+                                      bs.b[0], (uint8_t *)e->d_out.p, e->stream);
+                };
+                if ((st = time(count, launch, &best.matrix_rate))) return st;
+            }
             if (best.rate > 0) found.push_back(best);
         }
     }
@@ -142,9 +167,10 @@ extern "C" pgap_status pgap_autotune(pgap_engine *e, const uint32_t *bits, size_
             e->set_error("pgap_autotune: cannot write %s", path);
             return PGAP_E_ARG;
         }
-        fprintf(f, "# pgap tuning table: kind max_bits radix digits lanes blocks_cap tests_per_s\n");
+        fprintf(f, "# pgap tuning table: kind max_bits radix digits lanes blocks_cap tests_per_s matrix_tests_per_s\n");
         for (const TuneEntry &t : found)
-            fprintf(f, "%d %u %d %d %d %d %.1f\n", t.kind, t.bits, t.radix, t.digits, t.lanes, t.blocks_cap, t.rate);
+            fprintf(f, "%d %u %d %d %d %d %.1f %.1f\n", t.kind, t.bits, t.radix, t.digits, t.lanes, t.blocks_cap,
+                    t.rate, t.matrix_rate);
         fclose(f);
     }
     std::sort(found.begin(), found.end(), [](const TuneEntry &a, const TuneEntry &b) {

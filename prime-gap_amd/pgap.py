@@ -43,14 +43,14 @@ SIDES_BOTH, SIDES_PREV, SIDES_NEXT = 0, 1, 2
 
 def read_tuning(path: str) -> List[dict]:
     """Parse an autotuner table (the text format pgap_autotune writes)."""
-    keys = ("test", "bits", "radix", "digits", "lanes", "cap", "tests_per_s")
+    keys = ("test", "bits", "radix", "digits", "lanes", "cap", "tests_per_s", "matrix_tests_per_s")
     rows = []
     with open(path) as f:
         for line in f:
             if line.startswith("#") or not line.strip():
                 continue
             parts = line.split()
-            rows.append({k: (float(v) if k == "tests_per_s" else int(v)) for k, v in zip(keys, parts)})
+            rows.append({k: (float(v) if k.endswith("tests_per_s") else int(v)) for k, v in zip(keys, parts)})
     return rows
 
 
