@@ -2,6 +2,7 @@
 // first and run the kernels of mixed_impl.h (matrix-core numbers and one-lane
 // buckets side by side on two streams).
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "engine_impl.h"
@@ -106,17 +107,41 @@ static pgap_status mixed_once(pgap_engine *e, const uint32_t *words, const uint6
         bucket[(size_t)b].most = std::max(bucket[(size_t)b].most, bits);
         total_words = std::max<size_t>(total_words, offset[i] + limbs[i]);
     }
-    // One-lane buckets of more rows than the matrix cores test in the time of
-    // a round go to the persistent kernel in tiles of 64, widest first
-    // (order[1]); the other rows to the matrix cores by container, widest
-    // first (order[0]).
+    // Buckets below `cut` go to the persistent kernel in tiles of 64, widest
+    // first (order[1]); the other rows to the matrix cores by container, widest
+    // first (order[0]).  The one-lane tiles together take the widest one's time
+    // or the device's for their sum, whichever is more, so a narrower bucket
+    // costs nothing beside a wide one; rows on the matrix cores add up.  Chosen
+    // bucket by bucket instead (each against a round of its own), five buckets
+    // that each just stay below a round took 67.9 ms against 49.3 in tiles.
+    const double simds = 4.0 * e->num_cus;
+    int cut = 0;
+    double least = 0;
+    for (int c = N1; c >= 0; --c) {
+        if (c == 0 && !bucket[0].rows.empty() && bucket[0].most < kMatrixMinBits) break;
+        double longest = 0, tiles = 0, matrix = 0;
+        for (int b = 0; b < N1; ++b) {
+            const Bucket &k = bucket[(size_t)b];
+            if (k.rows.empty()) continue;
+            const double tile = kTileCycles[b] * k.most, rows = (double)k.rows.size();
+            if (b < c) {
+                longest = std::max(longest, tile);
+                tiles += std::ceil(rows / 64) * tile;
+            } else {
+                matrix += rows * kMixedMatrixCycles[find_matrix(KIND_FERMAT2, (int)k.most)->blocks] * k.most;
+            }
+        }
+        const double time = std::max(longest, tiles / simds) + matrix / simds;
+        if (c == N1 || time < least) {
+            least = time;
+            cut = c;
+        }
+    }
     std::vector<uint32_t> order[2], container[kMixedContainers];
     std::vector<uint8_t> tile_bucket;
     for (int b = N1; b >= 0; --b) {
         const Bucket &k = bucket[(size_t)b];
-        const MatrixVariant *mx = k.rows.empty() ? nullptr : find_matrix(KIND_FERMAT2, (int)k.most);
-        if (b == N1 || (mx && k.most >= kMatrixMinBits &&
-                        k.rows.size() <= e->matrix_limit(MixedOneLane::digits[b], mx->blocks))) {
+        if (b >= cut) {
             for (size_t i = 0; i < k.rows.size(); ++i)
                 container[find_matrix(KIND_FERMAT2, (int)k.bits[i])->blocks - 1].push_back(k.rows[i]);
             continue;

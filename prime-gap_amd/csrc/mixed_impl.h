@@ -34,6 +34,13 @@ using MixedOneLane = Buckets<12, 26, 40, 56, 78>;
 constexpr int kMixedMaxBits = 28 * 160;
 constexpr int kMixedContainers = 9;  // matrix-core containers of 1 .. 9 blocks (mont_mf.h)
 static_assert(mf::max_bits(kMixedContainers) >= kMixedMaxBits, "the last container takes every number");
+// Cycles of a squaring, measured at the buckets' upper widths: of a one-lane tile
+// alone on its SIMD, by bucket (3311, 11001, 20056, 31691 and 38473 numbers of 330,
+// 720, 1110, 1560 and 2128 bits in 0.27, 2.0, 5.4, 14.2 and 46.8 ms), and of a SIMD
+// per number in mixed_mf_kernel, by blocks (the same numbers in 0.32, 2.3, 7.3, 16.8
+// and 40.9 ms: two wavefronts per SIMD cost the narrow ones 20 to 30%).
+constexpr double kTileCycles[MixedOneLane::n] = {2000, 6700, 11700, 21800, 52500};
+constexpr double kMixedMatrixCycles[6] = {0, 740, 700, 800, 840, 1250};
 
 // LDS park of the widest one-lane bucket (the last), one column per thread.
 constexpr size_t kMixedParkBytes =
