@@ -1002,7 +1002,8 @@ class Scanner {
         // sides that will scan this round (m's waiting for confirmations do not)
         const uint32_t sides = (uint32_t)std::min<uint64_t>(2ull * na, (uint64_t)last_scanning + 2ull * admitted_last);
         const MatrixVariant *mx = nullptr;  // of the round's strong-PRP and Fermat rows
-        if (!e->forced() && ((cf.v->lanes > 1 && !cf.tuned_group()) || sides <= LATENCY_SIDES))
+        // a cap on the occupancy is for the one-lane rounds
+        if (!e->opt.lanes_per_number && !e->opt.radix && ((cf.v->lanes > 1 && !cf.tuned_group()) || sides <= LATENCY_SIDES))
             mx = find_matrix(conf.n ? KIND_SPRP : KIND_FERMAT2, (int)bits);
         const Variant *vf = cf.v, *vc = cc.v;
         if (vc && !vc->scan) {
@@ -1067,7 +1068,7 @@ class Scanner {
                 lres = LUCAS_LANES;
             } else if (nluc) {
                 // one kernel for every round's Lucas tests, whatever a table has for batches
-                if (!e->forced()) lc.mx = find_matrix(KIND_LUCAS, (int)bits);
+                if (!e->opt.lanes_per_number && !e->opt.radix) lc.mx = find_matrix(KIND_LUCAS, (int)bits);
                 if (!lc.mx && (st = e->plan(KIND_LUCAS, bits, none, &lc))) return st;
                 lres = resident < resident_full ? (lc.mx ? LUCAS_LANES : (uint32_t)lc.lane.v->lanes) : 0u;
             }
