@@ -66,6 +66,15 @@ constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may a
 // Numbers too wide for one lane run on the matrix cores whatever their count,
 // unless a tuning table has a lane group faster.
 constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
+// A one-lane round of narrow numbers is short too, and without a strong Lucas
+// test (which is ten times longer on a lane group) it is the matrix round that
+// has little to gain: fewer sides without confirmations, none below 256 bits.
+// Scans of 1 / 256 / 500 m's, ms, one lane against matrix: 101# (135 bits) with
+// strong PRP confirmations 0.21 / 1.3 / 2.2 against 0.23 / 1.6 / 2.7; without any
+// 251# (345 bits) 0.43 / 1.8 / 2.6 against 0.23 / 1.7 / 2.9, 503# (705) 1.7 / - / 6.2
+// against 0.43 / - / 5.3; with Baillie-PSW 101# 0.72 / 2.7 / 3.8 against 0.28 / 1.5 / 2.4.
+constexpr uint32_t LATENCY_SIDES_NARROW = 512;  // no confirmation, one-lane variant below
+constexpr int LATENCY_NARROW_DIGITS = 26;       // ... so many digits
 // Full and held: 4 and 2 take 46.5 ms for 300 m's of 1511#, 2 and 2 46.8, 3 and
 // 2 49, 4 and 1 54.
 constexpr uint32_t MATRIX_WAVES = 4;      // wavefronts per SIMD in a full matrix round
@@ -1001,9 +1010,13 @@ class Scanner {
         if (conf.n && (st = e->pick(KIND_SPRP, bits, &cc))) return st;
         // sides that will scan this round (m's waiting for confirmations do not)
         const uint32_t sides = (uint32_t)std::min<uint64_t>(2ull * na, (uint64_t)last_scanning + 2ull * admitted_last);
+        const uint32_t few = lucas                                             ? LATENCY_SIDES
+                             : bits < kMatrixMinBits                           ? 0u
+                             : !conf.n && cf.v->digits < LATENCY_NARROW_DIGITS ? LATENCY_SIDES_NARROW
+                                                                               : LATENCY_SIDES;
         const MatrixVariant *mx = nullptr;  // of the round's strong-PRP and Fermat rows
         // a cap on the occupancy is for the one-lane rounds
-        if (!e->opt.lanes_per_number && !e->opt.radix && ((cf.v->lanes > 1 && !cf.tuned_group()) || sides <= LATENCY_SIDES))
+        if (!e->opt.lanes_per_number && !e->opt.radix && ((cf.v->lanes > 1 && !cf.tuned_group()) || sides <= few))
             mx = find_matrix(conf.n ? KIND_SPRP : KIND_FERMAT2, (int)bits);
         const Variant *vf = cf.v, *vc = cc.v;
         if (vc && !vc->scan) {

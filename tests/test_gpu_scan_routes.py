@@ -35,3 +35,15 @@ def test_an_occupancy_cap_keeps_the_matrix_rounds(confirm):
     assert row == capped_row == lane_row == (want["prev_p"], want["next_p"], want["p_tests"], want["n_tests"])
     assert issued < 4000 and lane >= 2 * len(xs) - 200
     assert abs(capped - issued) < 1000  # the same rounds; a Lucas test may end in another one
+
+
+@pytest.mark.parametrize("P,confirm,matrix", [(101, pgap.CONFIRM_BPSW, True), (101, pgap.CONFIRM_SPRP2, False),
+                                              (101, pgap.CONFIRM_NONE, False), (251, pgap.CONFIRM_SPRP2, True),
+                                              (251, pgap.CONFIRM_NONE, True)])
+def test_narrow_numbers_without_lucas_tests_stay_on_one_lane(P, confirm, matrix):
+    d, SL, m = 210, 8000, 101
+    xs = offsets(P, d, m, SL)
+    row, issued = scan(P, d, SL, m, xs, confirm)
+    want = ol.test_interval(P, d, m, SL, xs, xs, kind=0)
+    assert row == (want["prev_p"], want["next_p"], want["p_tests"], want["n_tests"])
+    assert issued < 4000 if matrix else issued >= 2 * len(xs) - 200
