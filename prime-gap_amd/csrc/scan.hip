@@ -66,15 +66,11 @@ constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may a
 // Numbers too wide for one lane run on the matrix cores whatever their count,
 // unless a tuning table has a lane group faster.
 constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
-// A one-lane round of narrow numbers is short too, and without a strong Lucas
-// test (which is ten times longer on a lane group) it is the matrix round that
-// has little to gain: fewer sides without confirmations, none below 256 bits.
-// Scans of 1 / 256 / 500 m's, ms, one lane against matrix: 101# (135 bits) with
-// strong PRP confirmations 0.21 / 1.3 / 2.2 against 0.23 / 1.6 / 2.7; without any
-// 251# (345 bits) 0.43 / 1.8 / 2.6 against 0.23 / 1.7 / 2.9, 503# (705) 1.7 / - / 6.2
-// against 0.43 / - / 5.3; with Baillie-PSW 101# 0.72 / 2.7 / 3.8 against 0.28 / 1.5 / 2.4.
-constexpr uint32_t LATENCY_SIDES_NARROW = 512;  // no confirmation, one-lane variant below
-constexpr int LATENCY_NARROW_DIGITS = 26;       // ... so many digits
+// Below 256 bits a one-lane round is as short, and only the strong Lucas tests gain
+// (ten times longer on a lane group): scans of 1 / 8 m's of 101# (135 bits), ms, one
+// lane against matrix, 0.12 / 0.23 against 0.14 / 0.27 without confirmations, 0.21 /
+// 0.34 against 0.23 / 0.38 with strong PRP ones, 0.70 / 1.30 against 0.28 / 0.44 with
+// Baillie-PSW.  At 345 bits (251#) one m takes 0.38 against 0.22 without any.
 // Full and held: 4 and 2 take 46.5 ms for 300 m's of 1511#, 2 and 2 46.8, 3 and
 // 2 49, 4 and 1 54.
 constexpr uint32_t MATRIX_WAVES = 4;      // wavefronts per SIMD in a full matrix round
@@ -1010,10 +1006,7 @@ class Scanner {
         if (conf.n && (st = e->pick(KIND_SPRP, bits, &cc))) return st;
         // sides that will scan this round (m's waiting for confirmations do not)
         const uint32_t sides = (uint32_t)std::min<uint64_t>(2ull * na, (uint64_t)last_scanning + 2ull * admitted_last);
-        const uint32_t few = lucas                                             ? LATENCY_SIDES
-                             : bits < kMatrixMinBits                           ? 0u
-                             : !conf.n && cf.v->digits < LATENCY_NARROW_DIGITS ? LATENCY_SIDES_NARROW
-                                                                               : LATENCY_SIDES;
+        const uint32_t few = lucas || bits >= kMatrixMinBits ? LATENCY_SIDES : 0u;
         const MatrixVariant *mx = nullptr;  // of the round's strong-PRP and Fermat rows
         // a cap on the occupancy is for the one-lane rounds
         if (!e->opt.lanes_per_number && !e->opt.radix && ((cf.v->lanes > 1 && !cf.tuned_group()) || sides <= few))
