@@ -202,7 +202,15 @@ pgap_status pgap_engine::pick(int kind, uint32_t bits, Choice *out) {
 // keeps the lane kernels, and so does a tuning table whose entry is a lane group
 // unless it has the matrix cores faster; a one-lane entry's remainders follow
 // the rule above (the table holds rates of full launches, not latencies).
-constexpr uint32_t kMatrixCycles[6] = {0, 400, 480, 590, 710, 1110};  // by container
+//
+// kMatrixCycles, by container, so that a width's remainder at the limit takes no
+// longer than a round: there a squaring takes 490 (280 and 330 bits) to 614 (256), 460
+// (705 to 970) to 556 (480), 582 (1108) to 627 (1000), 660 to 671 and 1089 to 1110 cycles
+// per SIMD and number, and one lane 4.1 (640 bits, 1000) to 5.8 for its
+// instruction.  Over 36 widths the limit's rows take 0.68 to 1.00 of a round, and 1.04
+// at 547 bits (6474 rows, the second half of their 4096 wavefronts' places
+// empty); with 480 and 590 for two and three blocks 640 bits took 1.06, 1000 bits 1.04.
+constexpr uint32_t kMatrixCycles[6] = {0, 400, 515, 670, 710, 1110};
 
 uint32_t pgap_engine::matrix_limit(int digits, int blocks) const {
     const uint64_t L = (uint64_t)digits, simds = 4ull * (uint64_t)num_cus;
