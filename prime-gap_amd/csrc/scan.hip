@@ -47,6 +47,7 @@
 #include <thread>
 #include <vector>
 
+#include "carry.h"
 #include "engine_impl.h"
 #include "waitq.h"
 
@@ -175,10 +176,7 @@ __global__ void scatter_kernel(const Upload *__restrict__ up, const uint32_t *__
 }
 
 // N = centre + x (side 1) or centre - x (side 0) as `w` words at o, by a
-// wavefront; the centre has cw words (zero above).  A lane passes a carry on
-// when its word is all ones (all zeros for a borrow), so adding the carry into
-// the lowest lane to the mask of such lanes flips exactly the lanes that
-// receive one.
+// wavefront, 64 words at a time (carry.h); the centre has cw words (zero above).
 __device__ __forceinline__ void write_n(const uint32_t *__restrict__ c, uint32_t cw, uint32_t side, uint32_t x,
                                         uint32_t *__restrict__ o, uint32_t w) {
     const uint32_t lane = threadIdx.x & 63u;
@@ -189,10 +187,10 @@ __device__ __forceinline__ void write_n(const uint32_t *__restrict__ c, uint32_t
         const bool low = j == 0;
         uint64_t pass = __ballot(!low && cj == (side ? ~0u : 0u));
         if (base == 0) in = (__ballot(low && (side ? first < x : cj < x)) & 1ull) << 1;
-        const uint64_t sum = pass + in, got = pass ^ sum;
-        const uint32_t one = (uint32_t)(got >> lane) & 1u;
+        const CarryChunk ch = carry_chunk(pass, in);
+        const uint32_t one = (uint32_t)(ch.got >> lane) & 1u;
         if (j < w) o[j] = low ? first : (side ? cj + one : cj - one);
-        in = sum < pass ? 1u : 0u;
+        in = ch.out;
     }
 }
 
