@@ -3,14 +3,13 @@
 // Reference counterpart: the reference compiles one container width per
 // binary (BITS, gap_test_gpu.cu:48-55, suggested ladder :669-686), so a
 // mixed workload either runs in the widest container or in one run per
-// width.  Here the numbers are grouped into size buckets.  Well-filled one-lane
-// buckets are cut into tiles of one wavefront (64 numbers), tiles are queued
+// width.  Here the numbers are grouped into size buckets.  The one-lane buckets
+// below a cut that the call's sizes give (mixed.hip) are divided into tiles of one wavefront (64 numbers), tiles are queued
 // widest first (longest-processing-time order), and a persistent grid of waves
 // pulls tiles from an atomic counter; each wave runs the radix-2^28 variant of
-// its tile's bucket.  Every wave leaves when the queue is empty.  The others,
-// numbers too wide for one lane and buckets of too few rows for it, run one
-// number per wavefront on the matrix cores, in one launch over all their
-// containers, widest first.  40% 705, 30% 2128 and 30% 4247 bits: 16411 numbers
+// its tile's bucket.  Every wave leaves when the queue is empty.  The others run one
+// number per wavefront on the matrix cores, over all their containers, widest
+// first.  40% 705, 30% 2128 and 30% 4247 bits: 16411 numbers
 // in 26.2 ms and 131072 in 191, against 93.2 and 309 with the wide ones on 8
 // lanes each and every other bucket in one-lane tiles; 2^19 narrow ones fill
 // the one-lane tiles and take 164 ms either way.

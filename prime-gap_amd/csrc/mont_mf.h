@@ -47,7 +47,11 @@ typedef int v4iu __attribute__((ext_vector_type(4), aligned(4)));
 constexpr uint32_t FLIP = 0x80808080u;
 // HB and HOFF of a width, see above.  Measured with both layouts, tests/s: 1108
 // bits (3 blocks) 3.67 -> 3.89 M with shared B fragments, 4247 (9) 232 -> 241 k;
-// 2128 (5) the same, where LW - 1 has the lower latency.
+// 2128 (5) the same, where LW - 1 has the lower latency; one and two blocks 2 to 6%
+// fewer (4096 of 450 bits 0.31 against 0.33 ms, 9000 of 705 1.33 against 1.39; one
+// number 1 to 4% sooner).  Four and eight blocks would need a tile more for their
+// word 16 KB, and at six and seven the high tiles from 64 reach past two (the
+// static assertion in Wave).
 constexpr bool shared_layout(int KB) { return KB == 3 || KB == 9; }
 template <int KB>
 struct Layout {

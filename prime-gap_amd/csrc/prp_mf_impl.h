@@ -26,7 +26,8 @@ __device__ __forceinline__ uint32_t prp_mf_test(const uint32_t *__restrict__ nw,
 }
 
 // Wavefronts per SIMD to schedule for: the narrow widths reach four without
-// spills (1108 bits: 8.23 ms for 32768 tests against 8.59 when asked for two),
+// spills (1108 bits: 4.34 ms for 16384 tests against 4.38 when asked for two, and
+// 0.58 for one against 0.56; one, two and four blocks the same within 1%),
 // the wide ones would spill (2128 bits: 36.0 against 30.8 ms).  Holding only the
 // loaded fragments of N and N^-1 and spreading them at each use takes 36 to 56
 // registers off, a wavefront more per SIMD, and is slower (16384 tests: 15.4 ->

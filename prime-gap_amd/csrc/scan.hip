@@ -65,15 +65,19 @@ constexpr uint32_t MAX_SLOTS = 1u << 16;  // m's in flight (the HBM budget may a
 // numbers a second (at 2128 bits 1.56 against 1.0 M/s, but in rounds of 42 ms)
 // once enough sides share a round that few of its tests run past a prime.
 // Numbers too wide for one lane run on the matrix cores whatever their count,
-// unless a tuning table has a lane group faster.
+// unless a tuning table has a lane group faster.  The threshold is met only near
+// capacity: 1511# with Poisson arrivals, p50 / p99 in ms for 512, 1024, 2048 and 4096
+// sides, 6.4 / 10 at 3000 m/s, 9.3 / 23 at 6600 and 27 / 81 at 8500 with each, 151 /
+// 331, 139 / 330, 118 / 381 and 111 / 469 at 10500; 9000 m's at once 11.4, 11.8, 12.1
+// and 12.0 k m/s.
 constexpr uint32_t LATENCY_SIDES = 1024;  // scanning sides at most
 // Below 256 bits a one-lane round is as short, and only the strong Lucas tests gain
 // (ten times longer on a lane group): scans of 1 / 8 m's of 101# (135 bits), ms, one
 // lane against matrix, 0.12 / 0.23 against 0.14 / 0.27 without confirmations, 0.21 /
 // 0.34 against 0.23 / 0.38 with strong PRP ones, 0.70 / 1.30 against 0.28 / 0.44 with
 // Baillie-PSW.  At 345 bits (251#) one m takes 0.38 against 0.22 without any.
-// Full and held: 4 and 2 take 46.5 ms for 300 m's of 1511#, 2 and 2 46.8, 3 and
-// 2 49, 4 and 1 54.
+// Wavefronts of a full and a held round, measured on 300 m's of 1511# at once: 4 and
+// 2 take 46.5 ms, 2 and 2 46.8, 3 and 2 49, 4 and 1 54.
 constexpr uint32_t MATRIX_WAVES = 4;      // wavefronts per SIMD in a full matrix round
 constexpr uint32_t MATRIX_WAVES_HELD = 2;  // ... while few sides scan
 constexpr uint32_t LUCAS_LANES = 128;     // of a strong Lucas test on the matrix cores

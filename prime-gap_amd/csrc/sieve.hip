@@ -194,7 +194,8 @@ __global__ void __launch_bounds__(1024) sieve_small_kernel(const uint64_t *__res
 // mod p: a pair is a hit only if the high word of v + margin is below that of
 // 2 SL 2^64 / p + 2 margin, two multiply-adds and a compare per pair instead
 // of two 64-bit Barrett reductions, and t = round(v p / 2^64) is exact while
-// 4 margin p < 2^63 (the caller checks it; m < 2^26 to 2 10^10).  Eight m's
+// 4 margin p < 2^63 (the caller asks for 2^62 over the batch's largest m: m < 2.8
+// 10^7 to 2 10^10; other batches take the exact route).  Eight m's
 // share a branch and a scalar load of the m's.  Bound by the multiply-add rate:
 // 200 m's of 1511# to 1e9 (10^10 pairs) take 1.19 ms against 14.0 with a Barrett
 // pair each, 8.5 10^12 pairs/s; 4096 m's 23 ms against 276.
